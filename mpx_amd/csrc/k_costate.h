@@ -20,7 +20,7 @@ constexpr int kCostateStages = 4;
 
 // One stage's data, lane (g, c): S_t rows 16 i + c, columns 16 k + 4 g + s;
 // dx_t entries 16 k + 4 g + s; dx_t, q_t, s_t, V_t, c_t rows 16 i + c;
-// r_t[c], du_t[c] (0 for t = N).
+// r_t and du_t of the lane's control 16 g + c (0 for t = N).
 template <int NT>
 struct CsStage {
   f4 S[NT][NT];
@@ -63,7 +63,7 @@ __device__ __forceinline__ void cs_load(CsStage<NT>& d, const Iter<float>& it, c
   }
   // stage N has no control: its r and du offsets fall past the records
   const int tu = t < N ? t : N - 1;
-  const int ou = t < N ? c * 4 : kOOB;
+  const int ou = t < N ? (16 * g + c) * 4 : kOOB;
   d.rr = rload(make_rsrc(ws.rh + ((size_t)b * N + tu) * m, m), ou);
   d.uu = rload(make_rsrc(ws.du + ((size_t)b * N + tu) * m, m), ou);
 }
@@ -72,8 +72,8 @@ template <int NT>
 __device__ __forceinline__ void cs_stage(const CsStage<NT>& d, const Ws<float>& ws, int b, int t, int n, int N,
                                          int g, int c, int lane) {
   const size_t st = (size_t)b * (N + 1) + t;
-  // q'dx and r'du on row 0 of the lanes
-  float df = g == 0 ? d.rr * d.uu : 0.f, dc = 0.f, lc = 0.f;
+  // q'dx on row 0 of the lanes, r'du one control per lane
+  float df = d.rr * d.uu, dc = 0.f, lc = 0.f;
 #pragma unroll
   for (int i = 0; i < NT; ++i) df += g == 0 ? d.qv[i] * d.xv[i] : 0.f;
   const rsrc_t rdv = make_rsrc(ws.dv + st * n, n);
@@ -122,6 +122,18 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WIDE ? 
     cs_load<NT, WIDE>(d0, it, ws, b, t + 2 < t1 ? t + 2 : t + 1, n, m, N, g, c);
     cs_stage<NT>(d1, ws, b, t + 1, n, N, g, c, lane);
   }
+}
+
+// One stage per wave, for the larger S_t of k_lqr_tile (two buffers of 16 or
+// 25 tiles would spill).
+template <int NT, bool WIDE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_costate_one(Prob<float> P, Iter<float> it, Ws<float> ws) {
+  const int t = blockIdx.x, b = blockIdx.y;
+  if (skip_instance(ws, b)) return;
+  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  CsStage<NT> d;
+  cs_load<NT, WIDE>(d, it, ws, b, t, P.n, P.m, P.N, g, c);
+  cs_stage<NT>(d, ws, b, t, P.n, P.N, g, c, lane);
 }
 
 }  // namespace mpxk

@@ -290,12 +290,12 @@ __device__ __forceinline__ float row16_bcast(float x) {
 // Z[J][:] *= id, Z[r][:] -= L[r][J] Z[J][:] for the rows r > J only (DPP row
 // masks).  Steps past m (pivot 1, zero column) change nothing that is read.
 template <int J, int KM>
-__device__ __forceinline__ void chol_step(f4& h, f4& z, const float (&fl)[16]) {
+__device__ __forceinline__ void chol_step(f4& h, f4& z, float fl) {
   constexpr int jg = J & 3, jv = J >> 2, pJ = 4 * (J & 3) + (J >> 2);
   const float hJ = row16_bcast<jg>(h[jv]);
   const float zJ = row16_bcast<jg>(z[jv]);
   const float a = fabsf(row_bcast<pJ>(hJ));
-  const float piv = fl[J] > a ? fl[J] : a;
+  const float piv = fl > a ? fl : a;
   const float id = __builtin_amdgcn_rsqf(piv);
   const float nid2 = -(id * id);
   const float nlc = hJ * nid2;   // -H[J][c] / a
@@ -326,7 +326,7 @@ __device__ __forceinline__ void chol_lower_inv(f4& h, f4& z, float floor) {
     constexpr int J = decltype(JJ)::value;
     fl[J] = floor * fabsf(rlane(h[J >> 2], 16 * (J & 3) + 4 * (J & 3) + (J >> 2)));
   });
-  static_for<0, 4 * KM>([&](auto JJ) { chol_step<decltype(JJ)::value, KM>(h, z, fl); });
+  static_for<0, 4 * KM>([&](auto JJ) { chol_step<decltype(JJ)::value, KM>(h, z, fl[decltype(JJ)::value]); });
 }
 
 // One stage's data in the interleaved order.

@@ -16,6 +16,7 @@
 #include "k_linearize.h"
 #include "k_lqr.h"
 #include "k_lqr_wave.h"
+#include "k_lqr_tile.h"
 #include "k_inst.h"
 #include "k_scan.h"
 #include "k_linesearch.h"
@@ -24,6 +25,7 @@
 #include "k_lin_mma.h"
 #include "k_fwd_tanh.h"
 #include "k_costate.h"
+#include "k_fwd_block.h"
 #include "k_adjoint.h"
 #include "k_misc.h"
 #include "k_caller.h"
@@ -90,8 +92,29 @@ bool wave_path(const mpxkkt_problem* pr, int flags, int P) {
          pr->n_eq <= 16 && pr->model != MPXKKT_MODEL_CALLER;
 }
 
+// The block-per-instance recursion on LDS operand tiles (k_lqr_tile): FP32 on
+// the matrix cores (flags bits 0 and 1 clear), one segment, n + 1 <= 80 and
+// m <= 32 (its LDS plan, 145 of 160 KB at the limit), n_eq <= 16, for what the
+// wave kernels do not take.  LQR phase against k_lqr_seq: 76 x 32 x 100 B = 8
+// 6.74 -> 1.13 ms, 76 x 32 x 50 p = 12 B = 256 3.75 -> 0.63 ms, 61 x 12 x 25
+// (caller) B = 64 1.12 -> 0.17 ms.  A caller's problem of one state tile (n <=
+// 15) stays on k_lqr_seq although this kernel is faster there too (13 x 12 x
+// 25 B = 64: 0.70 -> 0.085 ms): the quadruped's iterations on clipped penalties
+// amplify a last-digit change of the step to 1e-4 and more of the next iterate
+// (the two product forms of k_lqr_seq itself, flags bit 0, differ by as much in
+// half of the seeded batches), so its results keep their rounding.
+bool tile_path(const mpxkkt_problem* pr, int flags, int P) {
+  return pr->dtype == MPXKKT_F32 && (flags & 3) == 0 && P <= 1 && pr->n + 1 <= 80 && pr->m <= 32 &&
+         pr->n_eq <= 16 && !wave_path(pr, flags, P) && !(pr->model == MPXKKT_MODEL_CALLER && pr->n <= 15);
+}
+
+// whether the LQR solve works without the closed-loop maps F_t, f_t
+bool no_closed_loop(const mpxkkt_problem* pr, int flags, int P) {
+  return wave_path(pr, flags, P) || tile_path(pr, flags, P);
+}
+
 template <typename T>
-size_t carve(const mpxkkt_problem* pr, int P, bool wave, Ws<T>* ws, char* base) {
+size_t carve(const mpxkkt_problem* pr, int P, bool no_f, Ws<T>* ws, char* base) {
   const size_t B = pr->batch, n = pr->n, m = pr->m, N = pr->horizon, N1 = N + 1;
   size_t off = 0;
   auto take = [&](size_t cnt) -> T* {
@@ -112,8 +135,8 @@ size_t carve(const mpxkkt_problem* pr, int P, bool wave, Ws<T>* ws, char* base) 
   ws->s = take(B * N1 * n);
   ws->K = take(B * N * m * n);
   ws->k = take(B * N * m);
-  ws->F = take(wave ? 0 : B * N * n * n);
-  ws->f = take(wave ? 0 : B * N * n);
+  ws->F = take(no_f ? 0 : B * N * n * n);
+  ws->f = take(no_f ? 0 : B * N * n);
   ws->dx = take(B * N1 * n);
   ws->du = take(B * N * m);
   ws->dv = take(B * N1 * n);
@@ -139,13 +162,13 @@ size_t carve(const mpxkkt_problem* pr, int P, bool wave, Ws<T>* ws, char* base) 
 
 size_t workspace_bytes(const mpxkkt_problem* pr, const mpxkkt_params* prm) {
   const int P = effective_segments(pr, prm);
-  const bool wave = wave_path(pr, prm->flags, P);
+  const bool no_f = no_closed_loop(pr, prm->flags, P);
   if (pr->dtype == MPXKKT_F64) {
     Ws<double> w;
-    return carve<double>(pr, P, wave, &w, nullptr);
+    return carve<double>(pr, P, no_f, &w, nullptr);
   }
   Ws<float> w;
-  return carve<float>(pr, P, wave, &w, nullptr);
+  return carve<float>(pr, P, no_f, &w, nullptr);
 }
 
 mpxkkt_status check_view(const mpxkkt_view& v, const char* name, bool needed) {
@@ -358,6 +381,77 @@ mpxkkt_status run_scan(hipStream_t st, const mpxkkt_problem* pr, int nt, const P
 template <typename T>
 bool use_wave_lqr(const mpxkkt_problem* pr, const Prm<T>& R);
 
+template <typename T>
+bool use_tile_lqr(const mpxkkt_problem* pr, const Prm<T>& R) {
+  return IsF32<T>::value && tile_path(pr, R.flags, R.P);
+}
+
+inline bool al16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
+
+// f(integral_constant) for the tile counts of k_lqr_tile: NT = 1..5, MT = 1..2
+template <int LO, int HI, typename F>
+void with_count(int k, F&& f) {
+  if constexpr (LO < HI) {
+    if (k > LO) {
+      with_count<LO + 1, HI>(k, f);
+      return;
+    }
+  }
+  f(std::integral_constant<int, LO>{});
+}
+
+template <typename T>
+mpxkkt_status run_lqr_tile(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R,
+                           const Ws<T>& W, const LqrIn<T>& in) {
+  if constexpr (!IsF32<T>::value) {
+    return fail(MPXKKT_ERR_UNSUPPORTED, "tile LQR kernel is FP32 only");
+  } else {
+    mpxkkt_status s = MPXKKT_OK;
+    auto go = [&](auto nt, auto mt, auto mode) {
+      constexpr int NT = decltype(nt)::value, MT = decltype(mt)::value, MODE = decltype(mode)::value;
+      constexpr int NW = NT == 1 ? 4 : 8;
+      const size_t lds = (size_t)TileLds<T, NT, MT>::TOTAL * sizeof(T);
+      if ((s = prep_lds(k_lqr_tile<T, NT, MT, NW, MODE>, lds)) != MPXKKT_OK) return;
+      hipLaunchKernelGGL((k_lqr_tile<T, NT, MT, NW, MODE>), dim3(pr->batch), dim3(64 * NW), lds, st, P, R, W, in, 1);
+      s = launch_check("k_lqr_tile");
+    };
+    with_count<1, 5>((pr->n + 16) / 16, [&](auto nt) {
+      with_count<1, 2>((pr->m + 15) / 16, [&](auto mt) {
+        if (pr->model == MPXKKT_MODEL_CALLER) go(nt, mt, std::integral_constant<int, TILE_CALLER>{});
+        else go(nt, mt, std::integral_constant<int, TILE_A>{});
+      });
+    });
+    return s;
+  }
+}
+
+// after k_lqr_tile: the dx chain (k_fwd_block), then the costates over all stages
+template <typename T>
+mpxkkt_status run_fwd_tile(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Iter<T>& I,
+                           const Ws<T>& W, const LqrIn<T>& in) {
+  if constexpr (!IsF32<T>::value) {
+    return fail(MPXKKT_ERR_UNSUPPORTED, "tile LQR kernel is FP32 only");
+  } else {
+    const int nc = (pr->n + 15) / 16;
+    with_count<1, 5>(nc, [&](auto c) {
+      with_count<1, 2>((pr->m + 15) / 16, [&](auto mc) {
+        hipLaunchKernelGGL((k_fwd_block<T, decltype(c)::value, decltype(mc)::value>), dim3(pr->batch), dim3(512), 0,
+                           st, P, W, in);
+      });
+    });
+    mpxkkt_status s = launch_check("k_fwd_block");
+    if (s != MPXKKT_OK) return s;
+    const bool cw = (pr->n & 3) == 0 && al16(W.S) && al16(W.dx) && al16(W.qh);
+    with_count<1, 5>(nc, [&](auto c) {
+      constexpr int NC = decltype(c)::value;
+      const dim3 grid(pr->horizon + 1, pr->batch);
+      if (cw) hipLaunchKernelGGL((k_costate_one<NC, true>), grid, dim3(64), 0, st, P, I, W);
+      else hipLaunchKernelGGL((k_costate_one<NC, false>), grid, dim3(64), 0, st, P, I, W);
+    });
+    return launch_check("k_costate_one");
+  }
+}
+
 // k_fwd_wave for a stage-invariant B (cb) or not, with 128-bit tile loads when
 // n % 4 == 0 (wide)
 template <int NT>
@@ -408,8 +502,6 @@ bool mma_rows16(const mpxkkt_problem* pr) {
   return trial_rows16<T>(pr) && rows16(pr->xref, pr->n) && rows16(pr->uref, pr->m) &&
          (!pr->has_box || (rows16(pr->ulo, pr->m) && rows16(pr->uhi, pr->m)));
 }
-
-inline bool al16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
 
 // The tanh model on the wave path after k_linearize_mma (flags bit 3 clear:
 // it ran and wrote sd_t): the LQR kernels form f_x = I + h (A + kappa
@@ -486,6 +578,7 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
       return launch_check("k_costate_rows");
     }
   }
+  if (use_tile_lqr<T>(pr, R)) return run_fwd_tile<T>(st, pr, P, I, W, in);
   const int nt = 64;
   const size_t lds = stage_smem_elems<T>(pr->n, nt) * sizeof(T);
   mpxkkt_status s = prep_lds(k_fwd_stage<T>, lds);
@@ -633,6 +726,8 @@ mpxkkt_status run_lqr_m(hipStream_t st, const mpxkkt_problem* pr, int nt, const 
     if ((s = run_scan<T, MMAX>(st, pr, nt, P, R, I, W, in)) != MPXKKT_OK) return s;
   } else if (use_wave_lqr<T>(pr, R)) {
     return run_lqr_wave(st, pr, P, R, I, W, in);
+  } else if (use_tile_lqr<T>(pr, R)) {
+    return run_lqr_tile<T>(st, pr, P, R, W, in);
   } else {
     const size_t lds = ric_smem_elems<T>(pr->n, pr->m, pr->n_eq, nt, pr->M.ptr != nullptr) * sizeof(T);
     if ((s = prep_lds(k_lqr_seq<T, MMAX>, lds)) != MPXKKT_OK) return s;
@@ -833,7 +928,7 @@ mpxkkt_status sqp_iterate_t(hipStream_t st, const mpxkkt_problem* pr, const mpxk
                             bool gated = false) {
   const int Pseg = effective_segments(pr, prm);
   Ws<T> W;
-  carve<T>(pr, Pseg, wave_path(pr, prm->flags, Pseg), &W, static_cast<char*>(wsp));
+  carve<T>(pr, Pseg, no_closed_loop(pr, prm->flags, Pseg), &W, static_cast<char*>(wsp));
   if (!gated) W.run = nullptr;
   const Prob<T> P = make_prob<T>(pr);
   const Prm<T> R = make_prm<T>(prm, Pseg);
@@ -873,7 +968,7 @@ mpxkkt_status kkt_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_param
                     void* out, void* wsp) {
   Ws<T> W;
   const int Pseg = effective_segments(pr, prm);
-  carve<T>(pr, Pseg, wave_path(pr, prm->flags, Pseg), &W, static_cast<char*>(wsp));
+  carve<T>(pr, Pseg, no_closed_loop(pr, prm->flags, Pseg), &W, static_cast<char*>(wsp));
   const Prob<T> P = make_prob<T>(pr);
   const Prm<T> R = make_prm<T>(prm, 1);
   const Iter<T> I = make_iter<T>(it);
@@ -894,7 +989,7 @@ template <typename T>
 mpxkkt_status direction_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_params* prm,
                           mpxkkt_iterate* it, mpxkkt_direction* dir, void* wsp) {
   Ws<T> W;
-  carve<T>(pr, 1, false, &W, static_cast<char*>(wsp));
+  carve<T>(pr, 1, no_closed_loop(pr, prm->flags, 1), &W, static_cast<char*>(wsp));
   W.run = nullptr;
   const Prob<T> P = make_prob<T>(pr);
   const Prm<T> R = make_prm<T>(prm, 1);
@@ -918,7 +1013,7 @@ template <typename T>
 mpxkkt_status accept_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_params* prm, mpxkkt_iterate* it,
                        int L, const void* tg, const void* tf, mpxkkt_stats* so, void* wsp) {
   Ws<T> W;
-  carve<T>(pr, 1, false, &W, static_cast<char*>(wsp));
+  carve<T>(pr, 1, no_closed_loop(pr, prm->flags, 1), &W, static_cast<char*>(wsp));
   W.run = nullptr;
   const Prob<T> P = make_prob<T>(pr);
   Prm<T> R = make_prm<T>(prm, 1);
@@ -953,7 +1048,7 @@ template <typename T>
 mpxkkt_status srbd_iterate_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_srbd* model,
                              const mpxkkt_params* prm, mpxkkt_iterate* it, mpxkkt_stats* so, void* wsp) {
   Ws<T> W;
-  carve<T>(pr, 1, false, &W, static_cast<char*>(wsp));
+  carve<T>(pr, 1, no_closed_loop(pr, prm->flags, 1), &W, static_cast<char*>(wsp));
   W.run = nullptr;
   const Prob<T> P = make_prob<T>(pr);
   const Srbd<T> S = make_srbd<T>(model);
@@ -983,7 +1078,7 @@ mpxkkt_status solve_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_par
                       void* cost, void* cc, void* wsp, int32_t* launched) {
   Ws<T> W;
   const int Pseg = effective_segments(pr, prm);
-  carve<T>(pr, Pseg, wave_path(pr, prm->flags, Pseg), &W, static_cast<char*>(wsp));
+  carve<T>(pr, Pseg, no_closed_loop(pr, prm->flags, Pseg), &W, static_cast<char*>(wsp));
   const Prob<T> P = make_prob<T>(pr);
   const Iter<T> I = make_iter<T>(it);
   const int B = pr->batch, N1 = pr->horizon + 1;

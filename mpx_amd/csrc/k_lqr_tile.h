@@ -94,6 +94,14 @@ struct TileOps<float> {
   }
 };
 
+template <>
+struct TileOps<double> {
+  typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+  static __device__ __forceinline__ double bload(rsrc_t r, int off, int soff = 0) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
+  }
+};
+
 template <typename T>
 __device__ __forceinline__ rsrc_t tile_rsrc(const T* p, int nelem) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(p), (short)0, nelem * (int)sizeof(T), 0x00020000);

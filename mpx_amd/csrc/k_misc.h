@@ -135,13 +135,15 @@ __global__ void k_kkt_stage(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws) {
   if (tid == 0) ws.kpart[(size_t)b * N1 + t] = acc[0];
 }
 
+// square root of the stages' sum, one wave per instance (a thread per instance
+// walked its N + 1 entries one load after the other: 10.8 us at N = 50)
 template <typename T>
-__global__ void k_kkt_reduce(int B, int N1, const T* kpart, T* out) {
-  const int b = blockIdx.x * blockDim.x + threadIdx.x;
-  if (b >= B) return;
+__global__ void __launch_bounds__(64) k_kkt_reduce(int N1, const T* kpart, T* out) {
+  const int b = blockIdx.x;
   T s = 0;
-  for (int t = 0; t < N1; ++t) s += kpart[(size_t)b * N1 + t];
-  out[b] = dev_sqrt(s);
+  for (int t = threadIdx.x; t < N1; t += 64) s += kpart[(size_t)b * N1 + t];
+  s = wave_sum(s);
+  if (threadIdx.x == 0) out[b] = dev_sqrt(s);
 }
 
 // Row i of f(x_t, u_t) for the device model families (x, u of instance b).

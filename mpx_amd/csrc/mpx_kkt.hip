@@ -28,6 +28,8 @@
 #include "k_fwd_block.h"
 #include "k_adjoint.h"
 #include "k_misc.h"
+#include "k_eval.h"
+#include "k_eval_mma.h"
 #include "k_caller.h"
 #include "k_srbd.h"
 
@@ -963,6 +965,46 @@ mpxkkt_status sqp_iterate_t(hipStream_t st, const mpxkkt_problem* pr, const mpxk
   return s;
 }
 
+// k_eval_rows for n <= 80 (false: the general kernels), after k_eval_mma for the
+// stages t < N where its conditions hold (B = 1024, 36 x 12 x 50, p = 8: model
+// evaluation 180 -> 28 us, KKT residual 286 -> 53 us, a thread per row before
+// 812 and 343 us).  Stages per wave of
+// the row form: one until the stages fill the chip (a wave's stages run one
+// after the other), then four (the instance's matrices stay in L1).
+template <typename T, int WHAT>
+bool eval_rows(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R, const Iter<T>& I,
+               const Ws<T>& W, T* g, T* c) {
+  if (pr->n > 80) return false;
+  const int N1 = pr->horizon + 1;
+  int tbase = 0;
+  if constexpr (IsF32<T>::value) {
+    const int nt = mma_tiles<T>(pr, 0);
+    if (nt) {
+      const bool wide = mma_rows16<T>(pr) && al16(I.X) && al16(I.U) && al16(I.V) && al16(c) &&
+                        (WHAT != EVAL_KKT || !pr->has_box || al16(I.Ybox));
+      const dim3 grid((pr->horizon + 15) / 16, pr->batch);
+      with_count<1, 3>(nt, [&](auto k) {
+        constexpr int NT = decltype(k)::value;
+        if (wide) hipLaunchKernelGGL((k_eval_mma<NT, true, WHAT>), grid, dim3(64), 0, st, P, R, I, W, g, c);
+        else hipLaunchKernelGGL((k_eval_mma<NT, false, WHAT>), grid, dim3(64), 0, st, P, R, I, W, g, c);
+      });
+      tbase = pr->horizon;
+    }
+  }
+  const int spw = tbase == 0 && (long long)pr->batch * N1 >= 32768 ? 4 : 1;
+  const dim3 grid((N1 - tbase + kEvalWaves * spw - 1) / (kEvalWaves * spw), pr->batch);
+  with_count<1, 5>((pr->n + 15) / 16, [&](auto nc) {
+    constexpr int NC = decltype(nc)::value;
+    auto go = [&](auto mc) {
+      hipLaunchKernelGGL((k_eval_rows<T, NC, decltype(mc)::value, WHAT>), grid, dim3(64 * kEvalWaves), 0, st, P, R, I,
+                         W, g, c, spw, tbase);
+    };
+    if (pr->m <= 16) go(std::integral_constant<int, 1>{});
+    else go(std::integral_constant<int, 4>{});
+  });
+  return true;
+}
+
 template <typename T>
 mpxkkt_status kkt_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_params* prm, const mpxkkt_iterate* it,
                     void* out, void* wsp) {
@@ -972,14 +1014,16 @@ mpxkkt_status kkt_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_param
   const Prob<T> P = make_prob<T>(pr);
   const Prm<T> R = make_prm<T>(prm, 1);
   const Iter<T> I = make_iter<T>(it);
-  const int nt = k1_threads(pr->n);
-  const size_t lds = ((size_t)3 * pr->n + pr->m + nt) * sizeof(T);
-  mpxkkt_status s = prep_lds(k_kkt_stage<T>, lds);
-  if (s != MPXKKT_OK) return s;
-  hipLaunchKernelGGL(k_kkt_stage<T>, dim3(pr->horizon + 1, pr->batch), dim3(nt), lds, st, P, R, I, W);
+  mpxkkt_status s;
+  if (!eval_rows<T, EVAL_KKT>(st, pr, P, R, I, W, nullptr, nullptr)) {
+    const int nt = k1_threads(pr->n);
+    const size_t lds = ((size_t)3 * pr->n + pr->m + nt) * sizeof(T);
+    if ((s = prep_lds(k_kkt_stage<T>, lds)) != MPXKKT_OK) return s;
+    hipLaunchKernelGGL(k_kkt_stage<T>, dim3(pr->horizon + 1, pr->batch), dim3(nt), lds, st, P, R, I, W);
+  }
   if ((s = launch_check("k_kkt_stage")) != MPXKKT_OK) return s;
-  hipLaunchKernelGGL(k_kkt_reduce<T>, dim3((pr->batch + 255) / 256), dim3(256), 0, st, pr->batch,
-                     pr->horizon + 1, (const T*)W.kpart, static_cast<T*>(out));
+  hipLaunchKernelGGL(k_kkt_reduce<T>, dim3(pr->batch), dim3(64), 0, st, pr->horizon + 1, (const T*)W.kpart,
+                     static_cast<T*>(out));
   return launch_check("k_kkt_reduce");
 }
 
@@ -1091,7 +1135,8 @@ mpxkkt_status solve_t(hipStream_t st, const mpxkkt_problem* pr, const mpxkkt_par
   int done = 0;
   for (int i = 0; i < total; ++i) {
     if ((s = sqp_iterate_t<T>(st, pr, prm, it, so, wsp, true, true)) != MPXKKT_OK) return s;
-    hipLaunchKernelGGL(k_eval_partials<T>, dim3(N1, B), dim3(nt), 2 * nt * sizeof(T), st, P, I, W);
+    if (!eval_rows<T, EVAL_STOP>(st, pr, P, make_prm<T>(prm, Pseg), I, W, nullptr, nullptr))
+      hipLaunchKernelGGL(k_eval_partials<T>, dim3(N1, B), dim3(nt), 2 * nt * sizeof(T), st, P, I, W);
     if ((s = launch_check("k_eval_partials")) != MPXKKT_OK) return s;
     hipLaunchKernelGGL(k_stop<T>, gB, dim3(256), 0, st, B, N1, W, o->max_iter, (T)o->dcost_tol, (T)o->cc_tol,
                        iters, static_cast<T*>(cost), static_cast<T*>(cc));
@@ -1334,13 +1379,18 @@ mpxkkt_status mpxkkt_model_eval(void* stream, const mpxkkt_problem* prob, const 
   hipStream_t st = static_cast<hipStream_t>(stream);
   const int nt = k1_threads(prob->n);
   dim3 grid(prob->horizon + 1, prob->batch);
-  if (prob->dtype == MPXKKT_F64) {
-    hipLaunchKernelGGL(k_model_eval<double>, grid, dim3(nt), nt * sizeof(double), st, make_prob<double>(prob),
-                       (const double*)X, (const double*)U, (double*)g, (double*)c);
-  } else {
-    hipLaunchKernelGGL(k_model_eval<float>, grid, dim3(nt), nt * sizeof(float), st, make_prob<float>(prob),
-                       (const float*)X, (const float*)U, (float*)g, (float*)c);
-  }
+  auto launch = [&](auto zero) {
+    using T = decltype(zero);
+    const Prob<T> P = make_prob<T>(prob);
+    Iter<T> I = {};
+    I.X = static_cast<T*>(const_cast<void*>(X));   // read only
+    I.U = static_cast<T*>(const_cast<void*>(U));
+    if (!eval_rows<T, EVAL_MODEL>(st, prob, P, Prm<T>(), I, Ws<T>(), static_cast<T*>(g), static_cast<T*>(c)))
+      hipLaunchKernelGGL(k_model_eval<T>, grid, dim3(nt), nt * sizeof(T), st, P, static_cast<const T*>(X),
+                         static_cast<const T*>(U), static_cast<T*>(g), static_cast<T*>(c));
+  };
+  if (prob->dtype == MPXKKT_F64) launch(0.0);
+  else launch(0.0f);
   return launch_check("k_model_eval");
 }
 

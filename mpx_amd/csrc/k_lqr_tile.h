@@ -94,11 +94,42 @@ struct TileOps<float> {
   }
 };
 
+// (FP64: a result tile's register v of lane group g is row 4 v + g, not 4 g + v)
 template <>
 struct TileOps<double> {
+  typedef mpxk_f64x4 V4;
   typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+  static constexpr int PAD = 2;
+  static constexpr int RG = 4, RV = 1;
+  static __device__ __forceinline__ V4 mma(double a, double b, V4 c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ V4 load(const double* p) {
+    const mpxk_f64x2 a = reinterpret_cast<const mpxk_f64x2*>(p)[0], b = reinterpret_cast<const mpxk_f64x2*>(p)[1];
+    return V4{a[0], a[1], b[0], b[1]};
+  }
+  static __device__ __forceinline__ void store4(double* p, const V4& x) {
+    reinterpret_cast<mpxk_f64x2*>(p)[0] = mpxk_f64x2{x[0], x[1]};
+    reinterpret_cast<mpxk_f64x2*>(p)[1] = mpxk_f64x2{x[2], x[3]};
+  }
+  static __device__ __forceinline__ void store_col(double* p, int g, const V4& x) {
+#pragma unroll
+    for (int v = 0; v < 4; ++v) p[4 * v + g] = x[v];
+  }
+  static __device__ __forceinline__ V4 load_col(const double* p, int g) {
+    return V4{p[g], p[4 + g], p[8 + g], p[12 + g]};
+  }
+  static __device__ __forceinline__ int pos(int g, int v) { return 4 * v + g; }
   static __device__ __forceinline__ double bload(rsrc_t r, int off, int soff = 0) {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, 0));
+  }
+  static __device__ __forceinline__ V4 bload4(rsrc_t r, int off, int soff) {
+    const mpxk_f64x2 a = __builtin_bit_cast(mpxk_f64x2, __builtin_amdgcn_raw_buffer_load_b128(r, off, soff, 0));
+    const mpxk_f64x2 b = __builtin_bit_cast(mpxk_f64x2, __builtin_amdgcn_raw_buffer_load_b128(r, off + 16, soff, 0));
+    return V4{a[0], a[1], b[0], b[1]};
+  }
+  static __device__ __forceinline__ void bstore(rsrc_t r, int off, int soff, double v) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, off, soff, 0);
   }
 };
 
@@ -129,7 +160,8 @@ struct TileLds {
   static constexpr int RD = RV + 16 * MT;
   static constexpr int QV = RD + 16 * MT;        // q by position
   static constexpr int EV = QV + 16 * NT;        // the unit diagonal taken out of A~ (0 or 1) by position
-  static constexpr int TOTAL = EV + 16 * NT;
+  static constexpr int NONE = EV + 16 * NT;      // what a block has past its matrix lands here, never read
+  static constexpr int TOTAL = NONE + 64;
 };
 
 // a b over KT k tiles; the even and the odd ones in two chains (half the
@@ -138,18 +170,23 @@ struct TileLds {
 template <typename T, int KT>
 __device__ __forceinline__ typename TileOps<T>::V4 tile_dot(const T* a, const T* b) {
   typedef TileOps<T> O;
+  constexpr int GR = sizeof(T) == 8 ? 2 : KT;   // k tiles whose operands are in registers at once
   typename O::V4 x[KT], y[KT], acc[2];
-#pragma unroll
-  for (int k = 0; k < KT; ++k) {
-    x[k] = O::load(a + 16 * k);
-    y[k] = O::load(b + 16 * k);
-  }
 #pragma unroll
   for (int v = 0; v < 4; ++v) acc[0][v] = acc[1][v] = T(0);
 #pragma unroll
-  for (int s = 0; s < 4; ++s) {
+  for (int k0 = 0; k0 < KT; k0 += GR) {
 #pragma unroll
-    for (int k = 0; k < KT; ++k) acc[k & 1] = O::mma(x[k][s], y[k][s], acc[k & 1]);
+    for (int k = k0; k < KT && k < k0 + GR; ++k) {
+      x[k] = O::load(a + 16 * k);
+      y[k] = O::load(b + 16 * k);
+    }
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+#pragma unroll
+      for (int k = k0; k < KT && k < k0 + GR; ++k) acc[k & 1] = O::mma(x[k][s], y[k][s], acc[k & 1]);
+    }
+    if (GR < KT) __builtin_amdgcn_sched_barrier(0);
   }
   return KT > 1 ? acc[0] + acc[1] : acc[0];
 }
@@ -168,8 +205,11 @@ enum { TILE_A = 0, TILE_FX = 1, TILE_CALLER = 2 };
 // LDS as rows of Z and of Z'.  MT = 1: eight pivots each.  MT = 2 by blocks:
 // H00 = L00 L00', V = Z00 H01 (= L10'), then L11 L11' = H11 - V'V and
 // Z10 = -Z11 (V' Z00).  The pivot floors are those of H's own diagonal.
+template <typename T, int MT>
+struct TileFactor;
+
 template <int MT>
-struct TileFactor {
+struct TileFactor<float, MT> {
   static constexpr int LM = 16 * MT + 4;
   f4 h, z, d, u;   // the block under factorisation, its Z, its own H, -V' Z00
   template <int J0, int J1, int KM>
@@ -230,10 +270,62 @@ struct TileFactor {
   }
 };
 
+// FP64, m <= 16: lane k holds column k of H (identity past m) and of Z; pivot j
+// forms row j of L', divides by it and takes L[i][j] from lane i by readlane for
+// the trailing column and the forward substitution.
+template <>
+struct TileFactor<double, 1> {
+  static constexpr int LM = 18;
+  double h[16], z[16], hkk;
+  template <int J0, int J1>
+  __device__ __forceinline__ void steps(double floor, int k) {
+    static_for<J0, J1>([&](auto JJ) {
+      constexpr int J = decltype(JJ)::value;
+      const double d = dev_sqrt(floored_pivot(rlane(h[J], J), rlane(hkk, J), floor)), id = 1.0 / d;
+      const double lk = k > J ? h[J] * id : 0.0, zj = z[J] * id;
+      z[J] = zj;
+      static_for<J + 1, 16>([&](auto II) {
+        constexpr int i = decltype(II)::value;
+        const double lij = rlane(lk, i);
+        h[i] -= lij * lk;
+        z[i] -= lij * zj;
+      });
+    });
+  }
+  __device__ __forceinline__ void first(const mpxk_f64x4 (&H)[1][1], double* zr, double* zt, int ksm, double floor, int g,
+                                        int c) {
+    // through Z's place: rows and columns by position, column k = entry k
+#pragma unroll
+    for (int v = 0; v < 4; ++v) zr[(4 * v + g) * LM + c] = H[0][0][v];
+    wave_lds_sync();
+    const int k = 16 * g + c, kp = tile_pos(c);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      h[i] = zr[tile_pos(i) * LM + kp];
+      z[i] = k == i ? 1.0 : 0.0;
+      hkk = c == i ? h[i] : hkk;
+    }
+    wave_lds_sync();
+    steps<0, 8>(floor, k);
+  }
+  __device__ __forceinline__ void second(double* zr, double* zt, int ksm, double floor, int g, int c) {
+    const int k = 16 * g + c, kp = tile_pos(c);
+    if (ksm > 2) steps<8, 16>(floor, k);
+    if (g == 0) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        zr[tile_pos(i) * LM + kp] = z[i];
+        zt[kp * LM + tile_pos(i)] = z[i];
+      }
+    }
+  }
+};
+
 // n + 1 <= 16 NT (NT minimal), 16 (MT - 1) < m <= 16 MT, p <= 16.  Stores K~_t
 // and, with store_s, the upper tiles of S_t and s_t (k_costate_rows).  MODE:
 // TILE_FX forms f_x = I + h (A + kappa diag(sd_t) W) of the tanh model from
 // sd_t = ws.sdh; TILE_CALLER adds the caller's cross Hessian M_t (may be null).
+// FP64: m <= 16, n + 1 <= 64, both triangles of S_t.
 template <typename T, int NT, int MT, int NW, int MODE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
@@ -248,7 +340,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
   constexpr int T_C = MT == 2 ? T_B + NW - 3 : T_B;             // ... from T_C on in phase C
   constexpr int RC = T_C < NTT ? (NTT - T_C + NWK - 1) / NWK : 0;
   constexpr int RG = (NG + NW - 1) / NW;
-  static_assert(16 * NT * NT <= NTH && 16 * NT * MT <= NTH && 16 * NT <= 128 && NW >= 4, "a 4 x 4 block per thread");
+  static_assert(16 * NT * NT <= NTH, "a 4 x 4 block per thread");
   const int b = blockIdx.x;
   if (skip_instance(ws, b)) return;
   const int tid = threadIdx.x;
@@ -277,29 +369,32 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
   // ---- this thread's share of a stage's data: 4 x 4 blocks (rows g, 4 + g,
   // 8 + g, 12 + g of a k tile, four columns), a 128-bit LDS store per column.
   // The lanes of a 16 take the 4 x 4 blocks of a tile (64 bytes of each row;
-  // the columns' stores mostly in different banks); B~, and D and E in their one
-  // k tile, from the last threads down.
+  // the columns' stores mostly in different banks).  B~, D and E (in one k tile
+  // each) are the last waves' besides, each wave has one of them at most.
   const bool bconst = in.Bm.st == 0;
   const int na = (n + 15) >> 4, mb = (m + 15) >> 4;   // column tiles
-  const int tidr = NTH - 1 - tid;
+  constexpr int WB = (NT * MT + 3) / 4, WD = (NT + 3) / 4;
+  static_assert(WB + WD + 1 <= NW, "a wave for each small array");
+  const int role = w >= NW - WB ? 0 : w >= NW - WB - WD ? 1 : w == NW - WB - WD - 1 ? 2 : 3;   // B~, D, E, none
   struct Block {
     int off, lds[4];   // byte offset (kOOB: none), its columns' quads
   };
-  // (a column past the matrix lands in the padding of a row, which is never read)
-  auto block_of = [&](int e, int rows, int cols, int ld, int base, int stride, int width) {
+  auto block_of = [&](int e, int rows, int cols, int ld, int base, int stride) {
     Block k;
     const int kt = (e >> 4) / cols, ct = (e >> 4) - kt * cols, cb = e & 3, kq = (e >> 2) & 3, col = 16 * ct + 4 * cb;
     k.off = e >= 0 && kt < rows && col < ld ? ((16 * kt + kq) * ld + col) * ES : kOOB;
 #pragma unroll
     for (int j = 0; j < 4; ++j)   // column 4 cb + j: position + 4 j
       k.lds[j] = k.off != kOOB && col + j < ld ? base + (16 * ct + cb + 4 * j) * stride + 16 * kt + 4 * kq
-                                               : base + (tid & 15) * stride + width;
+                                               : X::NONE + 4 * (tid & 15);
     return k;
   };
-  const Block ka = block_of(tid, NT, na, n, X::AT, LD, 16 * NT), kb = block_of(tidr, NT, mb, m, X::BT, LD, 16 * NT);
-  const bool isd = w >= NW - 2;   // D in the last two waves, E in the one before
-  const Block kd = block_of(isd ? tidr : tidr - 128, 1, isd ? na : mb, isd ? n : m, isd ? X::DT : X::ET, LP, 16);
-  V4 ra[4], rb[4], rde[4], rcv;
+  const Block ka = block_of(tid, NT, na, n, X::AT, LD);
+  const int ts = tid - 64 * (role == 0 ? NW - WB : role == 1 ? NW - WB - WD : NW - WB - WD - 1);
+  const Block kb = role == 0 ? block_of(ts, NT, mb, m, X::BT, LD)
+                 : role == 1 ? block_of(ts, 1, na, n, X::DT, LP)
+                             : block_of(role == 2 ? ts : -1, 1, mb, m, X::ET, LP);
+  V4 ra[4], rb[4], rcv;
   V4 fa[MODE == TILE_FX ? 4 : 1], fw[MODE == TILE_FX ? 4 : 1];
   T rvr, rvd, rvq, rdg;
   const int sdo = (16 * ((tid >> 4) / na) + ((tid >> 2) & 3)) * ES;   // sd_t of a block's first row
@@ -321,8 +416,11 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
   };
   auto load_data = [&](int t) {
     // first what not every call has: the waits count the requests after it
-    if (!bconst && w >= NW - (NT * MT + 3) / 4) block_load(rb, tile_rsrc(pB + t * sB, n * m), kb.off, m);
-    if (p > 0 && w >= NW - 3) block_load(rde, tile_rsrc(isd ? pD + t * sD : pE + t * sE, isd ? p * n : p * m), kd.off, isd ? n : m);
+    if (role == 0 ? !bconst : role < 3 && p > 0) {
+      const T* q = role == 0 ? pB + t * sB : role == 1 ? pD + t * sD : pE + t * sE;
+      const int cols = role == 1 ? n : m, rows = role == 0 ? n : p;
+      block_load(rb, tile_rsrc(q, rows * cols), kb.off, cols);
+    }
     if constexpr (MODE == TILE_FX) {
       const rsrc_t rs = tile_rsrc(psd + (size_t)t * n, n);
 #pragma unroll
@@ -350,11 +448,12 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
     } else {
       block_store(ra, ka);
     }
-    if (!bconst && w >= NW - (NT * MT + 3) / 4) block_store(rb, kb);
-    if (p > 0 && w >= NW - 3) {
+    if (role == 0 ? !bconst : role < 3 && p > 0) {
+      if (role > 0) {
 #pragma unroll
-      for (int s = 0; s < 4; ++s) rde[s] *= sr;
-      block_store(rde, kd);
+        for (int s = 0; s < 4; ++s) rb[s] *= sr;
+      }
+      block_store(rb, kb);
     }
     if (tid < 4 * NT) O::store4(sm + X::AT + pn * LD + 4 * tid, rcv);   // column n: c
     if (tid < 16 * MT) {
@@ -448,7 +547,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
       fw[s] *= P.h * P.kappa;
     }
   }
-  if (bconst) {
+  if (bconst && role == 0) {
     block_load(rb, tile_rsrc(pB, n * m), kb.off, m);
     block_store(rb, kb);
   }
@@ -538,7 +637,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
       }
       lds_sync();
     }
-    TileFactor<MT> fac;
+    TileFactor<T, MT> fac;
     // C
     if (w == 0) {
       __builtin_amdgcn_s_setprio(3);
@@ -696,6 +795,11 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
             if (store_s) {
 #pragma unroll
               for (int v = 0; v < 4; ++v) O::bstore(rS, qo[s], v * srow, acc[v]);
+              if (sizeof(T) == 8 && i != j) {   // both triangles (k_fwd_stage)
+                const int qt = 16 * j + pc < n ? ((16 * j + pc) * n + 16 * i + O::RG * g) * ES : kOOB;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) O::bstore(rS, qt, v * O::RV * ES, acc[v]);
+              }
               if (j == NT - 1) {
 #pragma unroll
                 for (int v = 0; v < 4; ++v) O::bstore(rs, svo, (16 * i + O::RV * v) * ES, acc[v]);

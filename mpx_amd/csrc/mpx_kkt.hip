@@ -105,9 +105,13 @@ bool wave_path(const mpxkkt_problem* pr, int flags, int P) {
 // amplify a last-digit change of the step to 1e-4 and more of the next iterate
 // (the two product forms of k_lqr_seq itself, flags bit 0, differ by as much in
 // half of the seeded batches), so its results keep their rounding.
+// FP64 (v_mfma_f64): n + 1 <= 64 and m <= 16 (154 KB at the limit): 36 x 12 x 50
+// p = 8 B = 64 524 us (k_lqr_seq: 2690).
 bool tile_path(const mpxkkt_problem* pr, int flags, int P) {
-  return pr->dtype == MPXKKT_F32 && (flags & 3) == 0 && P <= 1 && pr->n + 1 <= 80 && pr->m <= 32 &&
-         pr->n_eq <= 16 && !wave_path(pr, flags, P) && !(pr->model == MPXKKT_MODEL_CALLER && pr->n <= 15);
+  if ((flags & 3) != 0 || P > 1 || pr->n_eq > 16) return false;
+  if (pr->dtype == MPXKKT_F64) return pr->n + 1 <= 64 && pr->m <= 16;
+  return pr->n + 1 <= 80 && pr->m <= 32 && !wave_path(pr, flags, P) &&
+         !(pr->model == MPXKKT_MODEL_CALLER && pr->n <= 15);
 }
 
 // whether the LQR solve works without the closed-loop maps F_t, f_t
@@ -385,7 +389,7 @@ bool use_wave_lqr(const mpxkkt_problem* pr, const Prm<T>& R);
 
 template <typename T>
 bool use_tile_lqr(const mpxkkt_problem* pr, const Prm<T>& R) {
-  return IsF32<T>::value && tile_path(pr, R.flags, R.P);
+  return tile_path(pr, R.flags, R.P);
 }
 
 inline bool al16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
@@ -405,44 +409,44 @@ void with_count(int k, F&& f) {
 template <typename T>
 mpxkkt_status run_lqr_tile(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R,
                            const Ws<T>& W, const LqrIn<T>& in) {
-  if constexpr (!IsF32<T>::value) {
-    return fail(MPXKKT_ERR_UNSUPPORTED, "tile LQR kernel is FP32 only");
-  } else {
-    mpxkkt_status s = MPXKKT_OK;
-    auto go = [&](auto nt, auto mt, auto mode) {
-      constexpr int NT = decltype(nt)::value, MT = decltype(mt)::value, MODE = decltype(mode)::value;
-      constexpr int NW = NT == 1 ? 4 : 8;
-      const size_t lds = (size_t)TileLds<T, NT, MT>::TOTAL * sizeof(T);
-      if ((s = prep_lds(k_lqr_tile<T, NT, MT, NW, MODE>, lds)) != MPXKKT_OK) return;
-      hipLaunchKernelGGL((k_lqr_tile<T, NT, MT, NW, MODE>), dim3(pr->batch), dim3(64 * NW), lds, st, P, R, W, in, 1);
-      s = launch_check("k_lqr_tile");
-    };
-    with_count<1, 5>((pr->n + 16) / 16, [&](auto nt) {
-      with_count<1, 2>((pr->m + 15) / 16, [&](auto mt) {
-        if (pr->model == MPXKKT_MODEL_CALLER) go(nt, mt, std::integral_constant<int, TILE_CALLER>{});
-        else go(nt, mt, std::integral_constant<int, TILE_A>{});
-      });
+  mpxkkt_status s = MPXKKT_OK;
+  auto go = [&](auto nt, auto mt, auto mode) {
+    constexpr int NT = decltype(nt)::value, MT = decltype(mt)::value, MODE = decltype(mode)::value;
+    constexpr int NW = NT == 1 ? 4 : 8;
+    const size_t lds = (size_t)TileLds<T, NT, MT>::TOTAL * sizeof(T);
+    if ((s = prep_lds(k_lqr_tile<T, NT, MT, NW, MODE>, lds)) != MPXKKT_OK) return;
+    hipLaunchKernelGGL((k_lqr_tile<T, NT, MT, NW, MODE>), dim3(pr->batch), dim3(64 * NW), lds, st, P, R, W, in, 1);
+    s = launch_check("k_lqr_tile");
+  };
+  with_count<1, IsF32<T>::value ? 5 : 4>((pr->n + 16) / 16, [&](auto nt) {
+    with_count<1, IsF32<T>::value ? 2 : 1>((pr->m + 15) / 16, [&](auto mt) {
+      if (pr->model == MPXKKT_MODEL_CALLER) go(nt, mt, std::integral_constant<int, TILE_CALLER>{});
+      else go(nt, mt, std::integral_constant<int, TILE_A>{});
     });
-    return s;
-  }
+  });
+  return s;
 }
 
 // after k_lqr_tile: the dx chain (k_fwd_block), then the costates over all stages
 template <typename T>
 mpxkkt_status run_fwd_tile(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Iter<T>& I,
                            const Ws<T>& W, const LqrIn<T>& in) {
-  if constexpr (!IsF32<T>::value) {
-    return fail(MPXKKT_ERR_UNSUPPORTED, "tile LQR kernel is FP32 only");
-  } else {
-    const int nc = (pr->n + 15) / 16;
-    with_count<1, 5>(nc, [&](auto c) {
-      with_count<1, 2>((pr->m + 15) / 16, [&](auto mc) {
-        hipLaunchKernelGGL((k_fwd_block<T, decltype(c)::value, decltype(mc)::value>), dim3(pr->batch), dim3(512), 0,
-                           st, P, W, in);
-      });
+  const int nc = (pr->n + 15) / 16;
+  with_count<1, IsF32<T>::value ? 5 : 4>(nc, [&](auto c) {
+    with_count<1, IsF32<T>::value ? 2 : 1>((pr->m + 15) / 16, [&](auto mc) {
+      hipLaunchKernelGGL((k_fwd_block<T, decltype(c)::value, decltype(mc)::value>), dim3(pr->batch), dim3(512), 0, st,
+                         P, W, in);
     });
-    mpxkkt_status s = launch_check("k_fwd_block");
-    if (s != MPXKKT_OK) return s;
+  });
+  mpxkkt_status s = launch_check("k_fwd_block");
+  if (s != MPXKKT_OK) return s;
+  if constexpr (!IsF32<T>::value) {
+    const int nt = 64;
+    const size_t lds = stage_smem_elems<T>(pr->n, nt) * sizeof(T);
+    if ((s = prep_lds(k_fwd_stage<T>, lds)) != MPXKKT_OK) return s;
+    hipLaunchKernelGGL(k_fwd_stage<T>, dim3(pr->horizon + 1, pr->batch), dim3(nt), lds, st, P, I, W);
+    return launch_check("k_fwd_stage");
+  } else {
     const bool cw = (pr->n & 3) == 0 && al16(W.S) && al16(W.dx) && al16(W.qh);
     with_count<1, 5>(nc, [&](auto c) {
       constexpr int NC = decltype(c)::value;

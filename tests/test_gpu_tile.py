@@ -90,3 +90,14 @@ def test_caller_linearisation(shape):
     for i, r in enumerate(refs):
         assert _rel(dX[i].double().cpu().numpy(), r["dX"]) < TOL["X"]
         assert _rel(dU[i].double().cpu().numpy(), r["dU"]) < TOL["U"]
+
+
+@pytest.mark.parametrize("wl,n,m,p", [
+    (3, 1, 1, 0), (3, 15, 16, 4), (4, 16, 8, 0), (3, 20, 9, 16), (4, 47, 16, 3), (3, 63, 5, 2), (1, 33, 12, 0),
+])
+def test_fp64(wl, n, m, p):
+    """FP64 (matrix cores): differs from the oracle by the order of sums."""
+    print(f"tile kernel FP64 wl={wl} n={n} m={m} p={p}", flush=True)
+    shape = dict(n=n, m=m, N=5) if wl == 1 else dict(n=n, m=m, N=5, p=p)
+    _check([syn.make_instance(wl, i, **shape) for i in range(2)], "tile" if wl == 1 else "rollout", 1 if wl == 1 else 2,
+           torch.float64, dict(X=1e-9, U=1e-8, V=1e-8))

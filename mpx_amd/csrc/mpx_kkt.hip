@@ -22,6 +22,7 @@
 #include "k_linesearch.h"
 #include "k_trials.h"
 #include "k_trials_mma.h"
+#include "k_rows_mma.h"
 #include "k_lin_mma.h"
 #include "k_fwd_tanh.h"
 #include "k_costate.h"
@@ -509,6 +510,53 @@ bool mma_rows16(const mpxkkt_problem* pr) {
          (!pr->has_box || (rows16(pr->ulo, pr->m) && rows16(pr->uhi, pr->m)));
 }
 
+// The matrix-core forms with the rows spread over a block's waves
+// (k_rows_mma.h), for what mma_tiles does not take: the tanh model with
+// stage-invariant A, W, B, Q, R, FP32 up to n = 80, m = 32, FP64 (the
+// linearisation) up to n = 64, m = 16; flags bit 4 clear, and the stage strides of the other views below
+// 2^22 entries (a block's 16 stages are addressed with 32-bit byte offsets).
+// Against the row-per-lane kernels: 76 x 32 x 50 p = 12 B = 256 linearisation
+// 334 -> 103 us, trials 221 -> 92.  Returns state tiles + 8 control tiles, 0
+// when they do not apply.
+template <typename T>
+int rows_tiles(const mpxkkt_problem* pr, int flags) {
+  if (pr->model != MPXKKT_MODEL_TANH || (flags & 16) != 0 || mma_tiles<T>(pr, flags) > 0) return 0;
+  if (pr->A.stage_stride != 0 || pr->W.stage_stride != 0 || pr->B.stage_stride != 0 || pr->Q.stage_stride != 0 ||
+      pr->R.stage_stride != 0)
+    return 0;
+  if (pr->n > (IsF32<T>::value ? 80 : 64) || pr->m > (IsF32<T>::value ? 32 : 16) || pr->n_eq > 64) return 0;
+  for (const mpxkkt_view* v : {&pr->xref, &pr->uref, &pr->D, &pr->E, &pr->e, &pr->ulo, &pr->uhi})
+    if (v->stage_stride > (1 << 22)) return 0;
+  return (pr->n + 15) / 16 + 8 * ((pr->m + 15) / 16);
+}
+
+// f with the tile counts of rows_tiles as constants (FP32: those mma_tiles leaves)
+template <typename T, typename F>
+void with_rows_tiles(int rt, F&& f) {
+  auto go = [&](auto nt, auto mt) { f(nt, mt); };
+  typedef std::integral_constant<int, 1> I1;
+  typedef std::integral_constant<int, 2> I2;
+  typedef std::integral_constant<int, 3> I3;
+  typedef std::integral_constant<int, 4> I4;
+  typedef std::integral_constant<int, 5> I5;
+  const int nt = rt & 7, mt = rt >> 3;
+  if constexpr (IsF32<T>::value) {
+    if (mt == 2) {
+      if (nt == 1) go(I1{}, I2{});
+      else if (nt == 2) go(I2{}, I2{});
+      else if (nt == 3) go(I3{}, I2{});
+      else if (nt == 4) go(I4{}, I2{});
+      else go(I5{}, I2{});
+      return;
+    }
+    if (nt == 5) return go(I5{}, I1{});
+  }
+  if (nt == 1) go(I1{}, I1{});
+  else if (nt == 2) go(I2{}, I1{});
+  else if (nt == 3) go(I3{}, I1{});
+  else go(I4{}, I1{});
+}
+
 // The tanh model on the wave path after k_linearize_mma (flags bit 3 clear:
 // it ran and wrote sd_t): the LQR kernels form f_x = I + h (A + kappa
 // diag(sd_t) W) where they use it and the linearisation does not write it.
@@ -651,6 +699,21 @@ mpxkkt_status run_linearize(hipStream_t st, const mpxkkt_problem* pr, const Prob
       }
       return launch_check("k_linearize_term");
     }
+  }
+  if (const int rt = caller ? 0 : rows_tiles<T>(pr, R.flags)) {
+    // FP32: 128-bit accesses of every row; FP64: of the Jacobian's rows (the
+    // descriptors' loads need dword alignment only, the workspace is aligned)
+    const bool wide = IsF32<T>::value ? mma_rows16<T>(pr) && al16(I.X) && al16(I.U) && al16(I.V) &&
+                                            (!pr->has_box || al16(I.Ybox))
+                                      : pr->n % 4 == 0;
+    const dim3 grid((pr->horizon + 15) / 16 + 1, pr->batch);
+    with_rows_tiles<T>(rt, [&](auto nt, auto mt) {
+      constexpr int NT = decltype(nt)::value, MT = decltype(mt)::value;
+      auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * (NT + MT)), 0, st, P, R, I, W); };
+      if (wide) go(k_linearize_rows<T, NT, MT, true>);
+      else go(k_linearize_rows<T, NT, MT, false>);
+    });
+    return launch_check("k_linearize_rows");
   }
   if (!caller && use_inst<T>(pr, false)) {
     const InstLds L = inst_lds(pr->n, pr->m, pr->horizon, pr->model == MPXKKT_MODEL_TANH, pr->Q.stage_stride == 0,
@@ -836,6 +899,19 @@ mpxkkt_status launch_trials(hipStream_t st, const TrialShape& ts, const Prob<T>&
 template <typename T>
 mpxkkt_status run_trials(hipStream_t st, const mpxkkt_problem* pr, const TrialShape& ts, const Prob<T>& P,
                          const Prm<T>& R, const Iter<T>& I, const Ws<T>& W, int j0, int j1) {
+  if constexpr (IsF32<T>::value) {   // FP64: bound by its tanh, k_trials is the faster one (36 x 12 x 50 B = 64: 36 us, here 44)
+    if (const int rt = rows_tiles<T>(pr, R.flags)) {
+      const bool wide = mma_rows16<T>(pr) && al16(I.X) && al16(I.U) && al16(I.V);
+      const dim3 grid((pr->horizon + 15) / 16 + 1, pr->batch);
+      with_rows_tiles<T>(rt, [&](auto nt, auto mt) {
+        constexpr int NT = decltype(nt)::value, MT = decltype(mt)::value;
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64 * (NT + MT)), 0, st, P, R, I, W, j0, j1); };
+        if (wide) go(k_trials_rows<T, NT, MT, true>);
+        else go(k_trials_rows<T, NT, MT, false>);
+      });
+      return launch_check("k_trials_rows");
+    }
+  }
   const int rows = std::max(pr->n, pr->n_eq);
   if (rows <= 64) return launch_trials<T, 1>(st, ts, P, R, I, W, j0, j1);
   if (rows <= 128) return launch_trials<T, 2>(st, ts, P, R, I, W, j0, j1);

@@ -16,6 +16,7 @@
 #include "k_linearize.h"
 #include "k_lqr.h"
 #include "k_lqr_wave.h"
+#include "k_lqr_small.h"
 #include "k_lqr_tile.h"
 #include "k_inst.h"
 #include "k_scan.h"
@@ -101,11 +102,10 @@ bool wave_path(const mpxkkt_problem* pr, int flags, int P) {
 // wave kernels do not take.  LQR phase against k_lqr_seq: 76 x 32 x 100 B = 8
 // 6.74 -> 1.13 ms, 76 x 32 x 50 p = 12 B = 256 3.75 -> 0.63 ms, 61 x 12 x 25
 // (caller) B = 64 1.12 -> 0.17 ms.  A caller's problem of one state tile (n <=
-// 15) stays on k_lqr_seq although this kernel is faster there too (13 x 12 x
-// 25 B = 64: 0.70 -> 0.085 ms): the quadruped's iterations on clipped penalties
-// amplify a last-digit change of the step to 1e-4 and more of the next iterate
-// (the two product forms of k_lqr_seq itself, flags bit 0, differ by as much in
-// half of the seeded batches), so its results keep their rounding.
+// 15) goes to k_lqr_small (small_path): the quadruped's iterations on clipped
+// penalties amplify a last-digit change of the step to 1e-4 and more of the
+// next iterate (the two product forms of k_lqr_seq, flags bit 0, differ by as
+// much in half of the seeded batches), so its results keep their rounding.
 // FP64 (v_mfma_f64): n + 1 <= 64 and m <= 16 (154 KB at the limit): 36 x 12 x 50
 // p = 8 B = 64 524 us (k_lqr_seq: 2690).
 bool tile_path(const mpxkkt_problem* pr, int flags, int P) {
@@ -113,6 +113,15 @@ bool tile_path(const mpxkkt_problem* pr, int flags, int P) {
   if (pr->dtype == MPXKKT_F64) return pr->n + 1 <= 64 && pr->m <= 16;
   return pr->n + 1 <= 80 && pr->m <= 32 && !wave_path(pr, flags, P) &&
          !(pr->model == MPXKKT_MODEL_CALLER && pr->n <= 15);
+}
+
+// One wave per instance (k_lqr_small): FP32, a caller's linearisation of one
+// state tile (n <= 15), one control tile, n_eq <= 16, one segment, flags bits 0
+// and 1 clear.  The results of k_lqr_seq bit for bit, in 133 us instead of 697
+// (13 x 12 x 25 B = 64).
+bool small_path(const mpxkkt_problem* pr, int flags, int P) {
+  return pr->dtype == MPXKKT_F32 && (flags & 3) == 0 && P <= 1 && pr->model == MPXKKT_MODEL_CALLER && pr->n <= 15 &&
+         pr->m <= 16 && pr->n_eq <= 16;
 }
 
 // whether the LQR solve works without the closed-loop maps F_t, f_t
@@ -797,6 +806,13 @@ mpxkkt_status run_lqr_m(hipStream_t st, const mpxkkt_problem* pr, int nt, const 
     return run_lqr_wave(st, pr, P, R, I, W, in);
   } else if (use_tile_lqr<T>(pr, R)) {
     return run_lqr_tile<T>(st, pr, P, R, W, in);
+  } else if (small_path(pr, R.flags, R.P)) {
+    if constexpr (IsF32<T>::value && MMAX == 16) {
+      auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(pr->batch), dim3(64), 0, st, P, R, W, in); };
+      if (pr->m <= 12) go(k_lqr_small<12>);
+      else go(k_lqr_small<16>);
+      return launch_check("k_lqr_small");
+    }
   } else {
     const size_t lds = ric_smem_elems<T>(pr->n, pr->m, pr->n_eq, nt, pr->M.ptr != nullptr) * sizeof(T);
     if ((s = prep_lds(k_lqr_seq<T, MMAX>, lds)) != MPXKKT_OK) return s;

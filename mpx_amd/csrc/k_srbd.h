@@ -257,149 +257,153 @@ __device__ __forceinline__ void penalty(T cv, T& val, T& d1, T& d2) {
   d2 = live ? a2 : T(0);
 }
 
-// stage cost l_t of quadruped_srbd_obj (t == N: terminal form)
+// The caller-form linearisation of the SRBD problem at (X_t, U_t), stage t =
+// blockIdx.x of instance blockIdx.y: A = f_x, B = f_u, fbar, Q, R, M (if given),
+// q, r, g (t < N); q_N, g_N, QN (t = N).  The first wave takes the cost, the
+// second the dynamics; the scalar chains (quaternion maps, the step and its
+// Jacobians) run on every lane alike, the entries of the cost's matrices are
+// spread over the lanes from LDS, each sum in the order of its index.  Bound by those scalar chains:
+// 13 x 12 x 25, B = 64 17 us; one thread per stage, which worked through every
+// entry of every matrix, 131.
 template <typename T>
-__device__ T srbd_cost(const T* W, const T* ref, const T* x, const T* u, bool term) {
-  T r[SRBD_RES];
-  for (int k = 0; k < 3; ++k) { r[k] = x[k] - ref[k]; r[6 + k] = x[7 + k] - ref[7 + k]; r[9 + k] = x[10 + k] - ref[10 + k]; }
-  quat_sub<T, false>(x + 3, ref + 3, r + 3, nullptr);
-  const int nr = term ? 12 : SRBD_RES;
-  if (!term)
-    for (int k = 0; k < 12; ++k) r[12 + k] = u[k];
-  T acc = 0;
-  for (int i = 0; i < nr; ++i) {
-    T wr = 0;
-    for (int j = 0; j < nr; ++j) wr += W[i * SRBD_RES + j] * r[j];
-    acc += r[i] * wr;
-  }
-  if (!term) {
-    for (int i = 0; i < 4; ++i) {
-      const T fx = u[3 * i], fy = u[3 * i + 1], fz = u[3 * i + 2];
-      const T cv = T(0.7) * fz - dev_sqrt(fx * fx + fy * fy + T(1e-2));
-      T v, d1, d2;
-      penalty(cv, v, d1, d2);
-      acc += v < T(1e-6) ? T(1e-6) : (v > T(1e6) ? T(1e6) : v);
-    }
-  }
-  return T(0.5) * acc;
-}
-
-// One thread per (stage t, instance b): the caller-form linearisation of the
-// SRBD problem at (X_t, U_t): A = f_x, B = f_u, fbar, Q, R, M (if given), q, r,
-// g (t < N); q_N, g_N, QN (t = N).
-template <typename T>
-__global__ void __launch_bounds__(64) k_srbd_linearize(Prob<T> P, Srbd<T> S, Iter<T> it) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(128) k_srbd_linearize(Prob<T> P, Srbd<T> S, Iter<T> it) {
+  constexpr int n = SRBD_N, m = SRBD_M, LW = SRBD_RES + 1;
+  const int t = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63;
   const int N = P.N, N1 = N + 1;
-  if (gid >= P.B * N1) return;
-  const int b = gid / N1, t = gid - b * N1;
   const bool term = t == N;
-  const T* x = it.X + ((size_t)b * N1 + t) * SRBD_N;
-  T u[SRBD_M];
-  for (int k = 0; k < SRBD_M; ++k) u[k] = term ? T(0) : it.U[((size_t)b * N + t) * SRBD_M + k];
-  const T* W = S.W.at(b, 0);
-  const T* ref = S.ref.at(b, t);
-  // residual and its state Jacobian (the quaternion block Jr, 3 x 4)
-  T r[SRBD_RES], Jr[12];
-  for (int k = 0; k < 3; ++k) { r[k] = x[k] - ref[k]; r[6 + k] = x[7 + k] - ref[7 + k]; r[9 + k] = x[10 + k] - ref[10 + k]; }
-  quat_sub<T, true>(x + 3, ref + 3, r + 3, Jr);
-  for (int k = 0; k < 12; ++k) r[12 + k] = u[k];
-  const int nr = term ? 12 : SRBD_RES;
-  // Wr = W r (rows 0..nr)
-  T Wr[SRBD_RES];
-  for (int i = 0; i < nr; ++i) {
-    T acc = 0;
-    for (int j = 0; j < nr; ++j) acc += W[i * SRBD_RES + j] * r[j];
-    Wr[i] = acc;
-  }
-  // J_x columns: residual row of state column c: p,dp,om identity; quat via Jr
-  // grad_x = J_x' W r
-  T gx[SRBD_N];
-  for (int c = 0; c < 3; ++c) { gx[c] = Wr[c]; gx[7 + c] = Wr[6 + c]; gx[10 + c] = Wr[9 + c]; }
-  for (int c = 0; c < 4; ++c) gx[3 + c] = Jr[c] * Wr[3] + Jr[4 + c] * Wr[4] + Jr[8 + c] * Wr[5];
-  T* qo = const_cast<T*>(P.q.at(b, t));
-  for (int c = 0; c < SRBD_N; ++c) qo[c] = gx[c];
-  // Q = J_x' W J_x: state column c maps to residual rows rowc (with weights)
-  // residual row index of state column c for the identity blocks
-  auto jx = [&](int rrow, int c) -> T {     // J_x[rrow][c]
-    if (c < 3) return rrow == c ? T(1) : T(0);
-    if (c < 7) return (rrow >= 3 && rrow < 6) ? Jr[(rrow - 3) * 4 + (c - 3)] : T(0);
-    if (c < 10) return rrow == c - 1 ? T(1) : T(0);
-    return rrow == c - 1 ? T(1) : T(0);
-  };
-  // WJ[i][c] = sum_r W[i][r] J_x[r][c] over the 12 state residual rows
-  T* Qo = const_cast<T*>(term ? P.QN.at(b, 0) : P.Q.at(b, t));
-  for (int c = 0; c < SRBD_N; ++c) {
-    T wj[12];
-    for (int i = 0; i < 12; ++i) {
-      T acc = 0;
-      for (int rr = 0; rr < 12; ++rr) acc += W[i * SRBD_RES + rr] * jx(rr, c);
-      wj[i] = acc;
+  __shared__ T sW[SRBD_RES * LW], x[n], u[m], ref[SRBD_REF], par[SRBD_PAR];
+  __shared__ T r[SRBD_RES], Jr[12], Wr[SRBD_RES], wj[12 * n], cone[4], d1[4], h[4], jf[12];
+  __shared__ T Fx[n * n], Fu[n * m];
+  {
+    const T* W = S.W.at(b, 0);
+    T w[5];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) w[k] = tid + 128 * k < SRBD_RES * SRBD_RES ? W[tid + 128 * k] : T(0);
+    if (tid < n) x[tid] = it.X[((size_t)b * N1 + t) * n + tid];
+    else if (tid >= 16 && tid < 16 + m) u[tid - 16] = term ? T(0) : it.U[((size_t)b * N + t) * m + tid - 16];
+    else if (tid >= 32 && tid < 32 + SRBD_REF) ref[tid - 32] = S.ref.at(b, t)[tid - 32];
+    else if (tid >= 64 && tid < 64 + SRBD_PAR) par[tid - 64] = term ? T(0) : S.par.at(b, t)[tid - 64];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      const int e = tid + 128 * k;
+      if (e < SRBD_RES * SRBD_RES) sW[e + e / SRBD_RES] = w[k];
     }
-    for (int c2 = 0; c2 < SRBD_N; ++c2) {
+  }
+  __syncthreads();
+
+  if (tid < 64) {
+    // residual and its state Jacobian (the quaternion block Jr, 3 x 4)
+    {
+      T rq[3], J[12];
+      quat_sub<T, true>(x + 3, ref + 3, rq, J);
+#pragma unroll
+      for (int k = 0; k < 12; ++k)
+        if (lane == k) Jr[k] = J[k];
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (lane == 3 + k) r[3 + k] = rq[k];
+      if (lane < 3) r[lane] = x[lane] - ref[lane];
+      if (lane >= 6 && lane < 12) r[lane] = x[lane + 1] - ref[lane + 1];
+      if (lane >= 12 && lane < SRBD_RES) r[lane] = u[lane - 12];
+    }
+    wave_lds_sync();
+    const int nr = term ? 12 : SRBD_RES;
+    // Wr = W r (rows 0..nr)
+    if (lane < nr) {
       T acc = 0;
-      for (int i = 0; i < 12; ++i) acc += jx(i, c2) * wj[i];
-      Qo[c2 * SRBD_N + c] = acc;
+      for (int j = 0; j < nr; ++j) acc += sW[lane * LW + j] * r[j];
+      Wr[lane] = acc;
+    }
+    // J_x[rrow][c]: p, dp, om identity; quat via Jr
+    auto jx = [&](int rrow, int c) -> T {
+      if (c < 3) return rrow == c ? T(1) : T(0);
+      if (c < 7) return (rrow >= 3 && rrow < 6) ? Jr[(rrow - 3) * 4 + (c - 3)] : T(0);
+      return rrow == c - 1 ? T(1) : T(0);
+    };
+    // wj[i][c] = sum_r W[i][r] J_x[r][c] over the 12 state residual rows
+    for (int e = lane; e < 12 * n; e += 64) {
+      const int i = e / n, c = e - i * n;
+      T acc = 0;
+      for (int rr = 0; rr < 12; ++rr) acc += sW[i * LW + rr] * jx(rr, c);
+      wj[e] = acc;
     }
     if (!term && P.M.p) {
-      // M[c2][j] = (J_x' W J_u)[c2][j] = sum_i J_x[i][c2] W[i][12 + j]
+      // M[c][j] = (J_x' W J_u)[c][j] = sum_i J_x[i][c] W[i][12 + j]
       T* Mo = const_cast<T*>(P.M.at(b, t));
-      for (int j = 0; j < SRBD_M; ++j) {
+      for (int e = lane; e < n * m; e += 64) {
+        const int c = e / m, j = e - c * m;
         T acc = 0;
-        for (int i = 0; i < 12; ++i) acc += jx(i, c) * W[i * SRBD_RES + 12 + j];
-        Mo[c * SRBD_M + j] = acc;
+        for (int i = 0; i < 12; ++i) acc += jx(i, c) * sW[i * LW + 12 + j];
+        Mo[e] = acc;
       }
     }
-  }
-  T* go = const_cast<T*>(P.g.at(b, t));
-  if (term) {
-    T acc = 0;
-    for (int i = 0; i < 12; ++i) acc += r[i] * Wr[i];
-    go[0] = T(0.5) * acc;
+    // friction cone values, Jacobian rows (3 nonzeros each), penalty derivatives
+    if (!term && lane < 4) {
+      const T fx = u[3 * lane], fy = u[3 * lane + 1], fz = u[3 * lane + 2];
+      const T rt = dev_sqrt(fx * fx + fy * fy + T(1e-2));
+      const T cv = T(0.7) * fz - rt;
+      T v, a1, a2;
+      penalty(cv, v, a1, a2);
+      const bool live = v > T(1e-6) && v < T(1e6);      // the outer clip of the objective
+      cone[lane] = v < T(1e-6) ? T(1e-6) : (v > T(1e6) ? T(1e6) : v);
+      d1[lane] = live ? a1 : T(0);
+      const T hc = a2 < T(1e-6) ? T(1e-6) : (a2 > T(1e6) ? T(1e6) : a2);
+      h[lane] = hc * ref[13 + lane];
+      jf[3 * lane] = -fx / rt;
+      jf[3 * lane + 1] = -fy / rt;
+      jf[3 * lane + 2] = T(0.7);
+    }
+    wave_lds_sync();
+    // grad_x = J_x' W r, Q = J_x' W J_x
+    T* qo = const_cast<T*>(P.q.at(b, t));
+    if (lane < 3) qo[lane] = Wr[lane];
+    else if (lane < 7) {
+      const int c = lane - 3;
+      qo[lane] = Jr[c] * Wr[3] + Jr[4 + c] * Wr[4] + Jr[8 + c] * Wr[5];
+    } else if (lane < n) qo[lane] = Wr[lane - 1];
+    T* Qo = const_cast<T*>(term ? P.QN.at(b, 0) : P.Q.at(b, t));
+    for (int e = lane; e < n * n; e += 64) {
+      const int c2 = e / n, c = e - c2 * n;
+      T acc = 0;
+      for (int i = 0; i < 12; ++i) acc += jx(i, c2) * wj[i * n + c];
+      Qo[e] = acc;
+    }
+    T* go = const_cast<T*>(P.g.at(b, t));
+    if (lane == 63) {
+      T acc = 0;
+      for (int i = 0; i < nr; ++i) acc += r[i] * Wr[i];
+      if (term) {
+        go[0] = T(0.5) * acc;
+      } else {
+        T pen = 0;
+        for (int i = 0; i < 4; ++i) pen += cone[i];
+        go[0] = T(0.5) * (acc + pen);
+      }
+    }
+    if (term) return;
+    // grad_u = (W r)[12:] + 1/2 J_f' d1 ; R = W[12:,12:] + J_f' diag(h) J_f
+    if (lane < m) {
+      const_cast<T*>(P.r.at(b, t))[lane] = Wr[12 + lane] + T(0.5) * jf[lane] * d1[lane / 3];
+    }
+    T* Ro = const_cast<T*>(P.R.at(b, t));
+    for (int e = lane; e < m * m; e += 64) {
+      const int j = e / m, k = e - j * m, fi = j / 3;
+      T v = sW[(12 + j) * LW + 12 + k];
+      if (fi == k / 3) v += jf[j] * h[fi] * jf[k];
+      Ro[e] = v;
+    }
     return;
   }
-  // friction cone values, Jacobian rows (3 nonzeros each), penalty derivatives
-  T pen = 0, d1[4], h[4], jf[4][3];
-  const T* contact = ref + 13;
-  for (int i = 0; i < 4; ++i) {
-    const T fx = u[3 * i], fy = u[3 * i + 1], fz = u[3 * i + 2];
-    const T rt = dev_sqrt(fx * fx + fy * fy + T(1e-2));
-    const T cv = T(0.7) * fz - rt;
-    T v, a1, a2;
-    penalty(cv, v, a1, a2);
-    const bool live = v > T(1e-6) && v < T(1e6);      // the outer clip of the objective
-    pen += v < T(1e-6) ? T(1e-6) : (v > T(1e6) ? T(1e6) : v);
-    d1[i] = live ? a1 : T(0);
-    const T hc = a2 < T(1e-6) ? T(1e-6) : (a2 > T(1e6) ? T(1e6) : a2);
-    h[i] = hc * contact[i];
-    jf[i][0] = -fx / rt;
-    jf[i][1] = -fy / rt;
-    jf[i][2] = T(0.7);
-  }
-  {
-    T acc = 0;
-    for (int i = 0; i < SRBD_RES; ++i) acc += r[i] * Wr[i];
-    go[0] = T(0.5) * (acc + pen);
-  }
-  // grad_u = (W r)[12:] + 1/2 J_f' d1 ; R = W[12:,12:] + J_f' diag(h) J_f
-  T* ro = const_cast<T*>(P.r.at(b, t));
-  T* Ro = const_cast<T*>(P.R.at(b, t));
-  for (int j = 0; j < SRBD_M; ++j) {
-    const int fi = j / 3, fk = j - 3 * fi;
-    ro[j] = Wr[12 + j] + T(0.5) * jf[fi][fk] * d1[fi];
-    for (int k = 0; k < SRBD_M; ++k) {
-      const int gi = k / 3, gk = k - 3 * gi;
-      T v = W[(12 + j) * SRBD_RES + 12 + k];
-      if (fi == gi) v += jf[fi][fk] * h[fi] * jf[gi][gk];
-      Ro[j * SRBD_M + k] = v;
-    }
-  }
-  // dynamics and Jacobians
-  const T* par = S.par.at(b, t);
+  if (term) return;
+
+  // dynamics and Jacobians, on every lane alike (the compiler fuses products
+  // with the sums that take them, so an entry's rounding depends on its whole
+  // expression: these stay one expression each)
   T* fo = const_cast<T*>(P.fbar.at(b, t));
   T xn[SRBD_N];
   srbd_step(S, x, u, par, xn);
-  for (int k = 0; k < SRBD_N; ++k) fo[k] = xn[k];
+  if (lane == 0)
+    for (int k = 0; k < SRBD_N; ++k) fo[k] = xn[k];
   const T dt = S.dt;
   const T* p = x;
   const T* quat = x + 3;
@@ -423,106 +427,197 @@ __global__ void __launch_bounds__(64) k_srbd_linearize(Prob<T> P, Srbd<T> S, Ite
   T Ji[9];
   for (int k = 0; k < 9; ++k) Ji[k] = S.Iinv[k] * dt;
   // fx rows of omega_next (10..12): [JiR'[f]x | Ji dR'w | 0 | I + Ji(-[om]x I + [I om]x)]
-  T Fx[SRBD_N * SRBD_N];
-  T Fu[SRBD_N * SRBD_M];
-  for (int k = 0; k < SRBD_N * SRBD_N; ++k) Fx[k] = 0;
-  for (int k = 0; k < SRBD_N * SRBD_M; ++k) Fu[k] = 0;
+  T Fo[3 * SRBD_N], Uo[3 * SRBD_M];
   T JiRt[9];
+#pragma unroll
   for (int i = 0; i < 3; ++i)
+#pragma unroll
     for (int j = 0; j < 3; ++j) {
       T acc = 0;
+#pragma unroll
       for (int k = 0; k < 3; ++k) acc += Ji[i * 3 + k] * Rm[j * 3 + k];
       JiRt[i * 3 + j] = acc;
     }
   T Iom[3];
+#pragma unroll
   for (int i = 0; i < 3; ++i) Iom[i] = S.I[i * 3] * om[0] + S.I[i * 3 + 1] * om[1] + S.I[i * 3 + 2] * om[2];
   const T sko[9] = {0, -om[2], om[1], om[2], 0, -om[0], -om[1], om[0], 0};
   const T skI[9] = {0, -Iom[2], Iom[1], Iom[2], 0, -Iom[0], -Iom[1], Iom[0], 0};
   T G[9];   // -[om]x I + [I om]x
+#pragma unroll
   for (int i = 0; i < 3; ++i)
+#pragma unroll
     for (int j = 0; j < 3; ++j) {
       T acc = 0;
+#pragma unroll
       for (int k = 0; k < 3; ++k) acc += sko[i * 3 + k] * S.I[k * 3 + j];
       G[i * 3 + j] = -acc + skI[i * 3 + j];
     }
+#pragma unroll
   for (int i = 0; i < 3; ++i) {
+#pragma unroll
     for (int j = 0; j < 3; ++j) {
       T a0 = 0, a1 = 0;
+#pragma unroll
       for (int k = 0; k < 3; ++k) { a0 += JiRt[i * 3 + k] * skf[k * 3 + j]; a1 += Ji[i * 3 + k] * G[k * 3 + j]; }
-      Fx[(10 + i) * SRBD_N + j] = a0;
-      Fx[(10 + i) * SRBD_N + 10 + j] = (i == j ? T(1) : T(0)) + a1;
+      Fo[i * SRBD_N + j] = a0;
+      Fo[i * SRBD_N + 7 + j] = 0;
+      Fo[i * SRBD_N + 10 + j] = (i == j ? T(1) : T(0)) + a1;
     }
+#pragma unroll
     for (int k = 0; k < 4; ++k) {
       T acc = 0;
+#pragma unroll
       for (int j = 0; j < 3; ++j) acc += Ji[i * 3 + j] * dRtw[k * 3 + j];
-      Fx[(10 + i) * SRBD_N + 3 + k] = acc;
+      Fo[i * SRBD_N + 3 + k] = acc;
     }
+#pragma unroll
     for (int f = 0; f < 4; ++f) {
       const T c = par[f];
       const T l[3] = {par[4 + 3 * f] - p[0], par[5 + 3 * f] - p[1], par[6 + 3 * f] - p[2]};
       const T skl[9] = {0, -l[2], l[1], l[2], 0, -l[0], -l[1], l[0], 0};
+#pragma unroll
       for (int j = 0; j < 3; ++j) {
         T acc = 0;
+#pragma unroll
         for (int k = 0; k < 3; ++k) acc += JiRt[i * 3 + k] * skl[k * 3 + j];
-        Fu[(10 + i) * SRBD_M + 3 * f + j] = acc * c;
+        Uo[i * SRBD_M + 3 * f + j] = acc * c;
       }
     }
-  }
-  // dp_next rows 7..9
-  for (int i = 0; i < 3; ++i) {
-    Fx[(7 + i) * SRBD_N + 7 + i] = T(1);
-    for (int f = 0; f < 4; ++f) Fu[(7 + i) * SRBD_M + 3 * f + i] = par[f] * dt / S.mass;
-  }
-  // p_new rows 0..2 = I (p) + dt * rows 7..9
-  for (int i = 0; i < 3; ++i) {
-    for (int j = 0; j < SRBD_N; ++j) Fx[i * SRBD_N + j] = (i == j ? T(1) : T(0)) + dt * Fx[(7 + i) * SRBD_N + j];
-    for (int j = 0; j < SRBD_M; ++j) Fu[i * SRBD_M + j] = dt * Fu[(7 + i) * SRBD_M + j];
   }
   // quat rows 3..6 = Jq (cols 3..6) + Jv * rows 10..12
   T Jq[16], Jv[12], qtmp[4];
   quat_integrate<T, true>(quat, xn + 10, dt, qtmp, Jq, Jv);
-  for (int i = 0; i < 4; ++i) {
-    for (int j = 0; j < SRBD_N; ++j) {
-      T acc = (j >= 3 && j < 7) ? Jq[i * 4 + (j - 3)] : T(0);
-      for (int k = 0; k < 3; ++k) acc += Jv[i * 3 + k] * Fx[(10 + k) * SRBD_N + j];
-      Fx[(3 + i) * SRBD_N + j] = acc;
-    }
-    for (int j = 0; j < SRBD_M; ++j) {
-      T acc = 0;
-      for (int k = 0; k < 3; ++k) acc += Jv[i * 3 + k] * Fu[(10 + k) * SRBD_M + j];
-      Fu[(3 + i) * SRBD_M + j] = acc;
+  if (lane == 0) {
+#pragma unroll
+    for (int e = 0; e < 3 * SRBD_N; ++e) Fx[10 * SRBD_N + e] = Fo[e];
+#pragma unroll
+    for (int e = 0; e < 3 * SRBD_M; ++e) Fu[10 * SRBD_M + e] = Uo[e];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+      for (int j = 0; j < SRBD_N; ++j) {
+        T acc = (j >= 3 && j < 7) ? Jq[i * 4 + (j - 3)] : T(0);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) acc += Jv[i * 3 + k] * Fo[k * SRBD_N + j];
+        Fx[(3 + i) * SRBD_N + j] = acc;
+      }
+#pragma unroll
+      for (int j = 0; j < SRBD_M; ++j) {
+        T acc = 0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) acc += Jv[i * 3 + k] * Uo[k * SRBD_M + j];
+        Fu[(3 + i) * SRBD_M + j] = acc;
+      }
     }
   }
+  // dp_next rows 7..9, and p_new rows 0..2 = I (p) + dt * rows 7..9
+  for (int e = lane; e < 3 * SRBD_N; e += 64) {
+    const int i = e / SRBD_N, j = e - i * SRBD_N;
+    const T v = j == 7 + i ? T(1) : T(0);
+    Fx[(7 + i) * SRBD_N + j] = v;
+    Fx[e] = (i == j ? T(1) : T(0)) + dt * v;
+  }
+  for (int e = lane; e < 3 * SRBD_M; e += 64) {
+    const int i = e / SRBD_M, q = e - i * SRBD_M;
+    const T v = q % 3 == i ? par[q / 3] * dt / S.mass : T(0);
+    Fu[(7 + i) * SRBD_M + q] = v;
+    Fu[e] = dt * v;
+  }
+  wave_lds_sync();
   T* Ao = const_cast<T*>(P.A.at(b, t));
   T* Bo = const_cast<T*>(P.Bm.at(b, t));
-  for (int k = 0; k < SRBD_N * SRBD_N; ++k) Ao[k] = Fx[k];
-  for (int k = 0; k < SRBD_N * SRBD_M; ++k) Bo[k] = Fu[k];
+  for (int k = lane; k < SRBD_N * SRBD_N; k += 64) Ao[k] = Fx[k];
+  for (int k = lane; k < SRBD_N * SRBD_M; k += 64) Bo[k] = Fu[k];
 }
 
-// One thread per (stage t, trial j, instance b): l_t and f at
-// x = X_t + a_j dX_t, u = U_t + a_j dU_t, a_j = a_max beta^j.
+// l_t and f at x = X_t + a_j dX_t, u = U_t + a_j dU_t, a_j = a_max beta^j, for
+// the L (N + 1) points of instance blockIdx.y: blocks [0, nc) take the cost l_t
+// of quadruped_srbd_obj (t == N: its terminal form) of 16 points, four lanes
+// each (lane s: rows s, s + 4, ... of W r, W in LDS; the terms are summed in
+// their order), the others the dynamics of 64 points, one lane each.  Bound by
+// the scalar chains of one point: 13 x 12 x 25, 10 trials, B = 64 7 us; a
+// thread per point for both, W from memory, 43.
+constexpr int kSrbdTrialPoints = 16;   // per cost block
 template <typename T>
-__global__ void __launch_bounds__(64) k_srbd_trials(Prob<T> P, Srbd<T> S, Iter<T> it, Ws<T> ws, T beta, int L) {
-  const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const int N = P.N, N1 = N + 1;
-  if (gid >= P.B * L * N1) return;
-  const int t = gid % N1, bj = gid / N1, j = bj % L, b = bj / L;
+__global__ void __launch_bounds__(64) k_srbd_trials(Prob<T> P, Srbd<T> S, Iter<T> it, Ws<T> ws, T beta, int L,
+                                                    int nc) {
+  constexpr int LW = SRBD_RES + 1;
+  __shared__ T sW[SRBD_RES * LW];
+  const int b = blockIdx.y, lane = threadIdx.x, N = P.N, N1 = N + 1;
   if (skip_instance(ws, b)) return;
+  const bool costs = (int)blockIdx.x < nc;
+  if (costs) {
+    const T* W = S.W.at(b, 0);
+    T w[9];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) w[k] = W[lane + 64 * k];
+#pragma unroll
+    for (int k = 0; k < 9; ++k) sW[lane + 64 * k + (lane + 64 * k) / SRBD_RES] = w[k];
+    __syncthreads();
+  }
+  // (points past the last one repeat it, nothing of theirs is stored)
+  const int id = costs ? blockIdx.x * kSrbdTrialPoints + (lane >> 2) : (blockIdx.x - nc) * 64 + lane;
+  const int pt = min(id, L * N1 - 1), j = pt / N1, t = pt - j * N1;
+  const bool term = t == N;
   T a = ws.lsp[(size_t)b * NLS + LS_AMAX];
   for (int q = 0; q < j; ++q) a *= beta;
-  const bool term = t == N;
   T x[SRBD_N], u[SRBD_M];
   const size_t ox = ((size_t)b * N1 + t) * SRBD_N;
+#pragma unroll
   for (int k = 0; k < SRBD_N; ++k) x[k] = it.X[ox + k] + a * ws.dx[ox + k];
-  const size_t ou = ((size_t)b * N + t) * SRBD_M;
+  const size_t ou = ((size_t)b * N + (term ? 0 : t)) * SRBD_M;
+#pragma unroll
   for (int k = 0; k < SRBD_M; ++k) u[k] = term ? T(0) : it.U[ou + k] + a * ws.du[ou + k];
-  ws.trial_g[((size_t)b * L + j) * N1 + t] = srbd_cost(S.W.at(b, 0), S.ref.at(b, t), x, u, term);
-  if (!term) {
+  if (!costs) {
+    if (id >= L * N1 || term) return;
     T xn[SRBD_N];
     srbd_step(S, x, u, S.par.at(b, t), xn);
     T* fo = ws.trial_f + (((size_t)b * L + j) * N + t) * SRBD_N;
+#pragma unroll
     for (int k = 0; k < SRBD_N; ++k) fo[k] = xn[k];
+    return;
   }
+  const int s = lane & 3;
+  const T* ref = S.ref.at(b, t);
+  T r[SRBD_RES];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    r[k] = x[k] - ref[k];
+    r[6 + k] = x[7 + k] - ref[7 + k];
+    r[9 + k] = x[10 + k] - ref[10 + k];
+  }
+  quat_sub<T, false>(x + 3, ref + 3, r + 3, nullptr);
+#pragma unroll
+  for (int k = 0; k < 12; ++k) r[12 + k] = u[k];   // 0 at the terminal stage: its rows and columns add nothing
+  T wr[6];
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    wr[k] = 0;
+#pragma unroll
+    for (int c = 0; c < SRBD_RES; ++c) wr[k] += sW[(s + 4 * k) * LW + c] * r[c];
+  }
+  T acc = 0;
+#pragma unroll
+  for (int k = 0; k < 6; ++k) {
+    acc += r[4 * k] * dpp_ror<0x00>(wr[k]);        // (quad_perm: the value of lane 0, 1, 2, 3 of the four)
+    acc += r[4 * k + 1] * dpp_ror<0x55>(wr[k]);
+    acc += r[4 * k + 2] * dpp_ror<0xaa>(wr[k]);
+    acc += r[4 * k + 3] * dpp_ror<0xff>(wr[k]);
+  }
+  // lane s: the penalty of foot s's friction cone
+  const T fx = s < 2 ? (s == 0 ? u[0] : u[3]) : (s == 2 ? u[6] : u[9]);
+  const T fy = s < 2 ? (s == 0 ? u[1] : u[4]) : (s == 2 ? u[7] : u[10]);
+  const T fz = s < 2 ? (s == 0 ? u[2] : u[5]) : (s == 2 ? u[8] : u[11]);
+  const T cv = T(0.7) * fz - dev_sqrt(fx * fx + fy * fy + T(1e-2));
+  T v, d1, d2;
+  penalty(cv, v, d1, d2);
+  const T pc = v < T(1e-6) ? T(1e-6) : (v > T(1e6) ? T(1e6) : v);
+  T full = acc + dpp_ror<0x00>(pc);
+  full += dpp_ror<0x55>(pc);
+  full += dpp_ror<0xaa>(pc);
+  full += dpp_ror<0xff>(pc);
+  if (s == 0 && id < L * N1) ws.trial_g[((size_t)b * L + j) * N1 + t] = T(0.5) * (term ? acc : full);
 }
 
 }  // namespace mpxk

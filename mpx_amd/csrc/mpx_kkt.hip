@@ -1195,15 +1195,16 @@ mpxkkt_status srbd_iterate_t(hipStream_t st, const mpxkkt_problem* pr, const mpx
   const Iter<T> I = make_iter<T>(it);
   const int B = pr->batch, N1 = pr->horizon + 1;
   const int L = std::max(1, std::min(prm->max_trials, MAX_TRIALS));
-  hipLaunchKernelGGL(k_srbd_linearize<T>, dim3((B * N1 + 63) / 64), dim3(64), 0, st, P, S, I);
+  hipLaunchKernelGGL(k_srbd_linearize<T>, dim3(N1, B), dim3(128), 0, st, P, S, I);
   mpxkkt_status s = launch_check("k_srbd_linearize");
   if (s != MPXKKT_OK) return s;
   mpxkkt_direction dir;
   dir.dX = nullptr;
   // the step stays in the workspace (direction_t exports only when asked)
   if ((s = direction_t<T>(st, pr, prm, it, &dir, wsp)) != MPXKKT_OK) return s;
-  hipLaunchKernelGGL(k_srbd_trials<T>, dim3((B * L * N1 + 63) / 64), dim3(64), 0, st, P, S, I, W,
-                     (T)prm->beta, L);
+  const int nc = (L * N1 + kSrbdTrialPoints - 1) / kSrbdTrialPoints;
+  hipLaunchKernelGGL(k_srbd_trials<T>, dim3(nc + (L * N1 + 63) / 64, B), dim3(64), 0, st, P, S, I, W, (T)prm->beta, L,
+                     nc);
   if ((s = launch_check("k_srbd_trials")) != MPXKKT_OK) return s;
   return accept_t<T>(st, pr, prm, it, L, W.trial_g, W.trial_f, so, wsp);
 }

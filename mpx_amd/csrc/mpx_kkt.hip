@@ -17,6 +17,7 @@
 #include "k_lqr.h"
 #include "k_lqr_wave.h"
 #include "k_lqr_small.h"
+#include "k_lqr_waves.h"
 #include "k_lqr_tile.h"
 #include "k_inst.h"
 #include "k_scan.h"
@@ -747,6 +748,14 @@ bool use_wave_lqr(const mpxkkt_problem* pr, const Prm<T>& R) {
   return IsF32<T>::value && wave_path(pr, R.flags, R.P);
 }
 
+// Up to this many instances the wave recursion takes NT + 1 waves per instance
+// (k_lqr_waves, the same bits), past it one: with 1024 SIMDs the extra waves are
+// free until each has one, then the one-wave form's fewer instructions win.
+// Iterations at 36 x 12 x 50 p = 8, one wave -> NT + 1: B = 1 453 -> 301 us, 256
+// 481 -> 332, 512 508 -> 420, 768 549 -> 608; 45 x 14 x 50 B = 512 648 -> 599, 768
+// 709 -> 827; 24 x 12 x 50 B = 512 315 -> 282, 1024 351 -> 425.
+constexpr int kWavesBatch = 512;
+
 template <typename T>
 mpxkkt_status run_lqr_wave(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R,
                            const Iter<T>& I, const Ws<T>& W, const LqrIn<T>& in) {
@@ -757,23 +766,25 @@ mpxkkt_status run_lqr_wave(hipStream_t st, const mpxkkt_problem* pr, const Prob<
     const bool cq = P.Q.st == 0 && P.R.st == 0 && in.Bm.st == 0;   // Q, B, R held for the whole recursion
     const dim3 gb(pr->batch);
     auto go = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, st, P, R, I, W, in); };
+    auto gow = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64 * (NT + 1)), 0, st, P, R, W, in); };
+    const bool waves = pr->batch <= kWavesBatch;
     if (cq) {
       // one instantiation per step count: the steps are unrolled matrix instructions
       auto cases = [&](auto FA, auto AS) {
         constexpr bool fa = decltype(FA)::value, as = decltype(AS)::value;
         switch (NT * 4 + ksn) {
-          case 5: go(k_lqr_wave<1, true, 1, fa, as>); break;
-          case 6: go(k_lqr_wave<1, true, 2, fa, as>); break;
-          case 7: go(k_lqr_wave<1, true, 3, fa, as>); break;
-          case 8: go(k_lqr_wave<1, true, 4, fa, as>); break;
-          case 9: go(k_lqr_wave<2, true, 1, fa, as>); break;
-          case 10: go(k_lqr_wave<2, true, 2, fa, as>); break;
-          case 11: go(k_lqr_wave<2, true, 3, fa, as>); break;
-          case 12: go(k_lqr_wave<2, true, 4, fa, as>); break;
-          case 13: go(k_lqr_wave<3, true, 1, fa, as>); break;
-          case 14: go(k_lqr_wave<3, true, 2, fa, as>); break;
-          case 15: go(k_lqr_wave<3, true, 3, fa, as>); break;
-          default: go(k_lqr_wave<3, true, 4, fa, as>); break;
+          case 5: waves ? gow(k_lqr_waves<1, true, 1, fa, as>) : go(k_lqr_wave<1, true, 1, fa, as>); break;
+          case 6: waves ? gow(k_lqr_waves<1, true, 2, fa, as>) : go(k_lqr_wave<1, true, 2, fa, as>); break;
+          case 7: waves ? gow(k_lqr_waves<1, true, 3, fa, as>) : go(k_lqr_wave<1, true, 3, fa, as>); break;
+          case 8: waves ? gow(k_lqr_waves<1, true, 4, fa, as>) : go(k_lqr_wave<1, true, 4, fa, as>); break;
+          case 9: waves ? gow(k_lqr_waves<2, true, 1, fa, as>) : go(k_lqr_wave<2, true, 1, fa, as>); break;
+          case 10: waves ? gow(k_lqr_waves<2, true, 2, fa, as>) : go(k_lqr_wave<2, true, 2, fa, as>); break;
+          case 11: waves ? gow(k_lqr_waves<2, true, 3, fa, as>) : go(k_lqr_wave<2, true, 3, fa, as>); break;
+          case 12: waves ? gow(k_lqr_waves<2, true, 4, fa, as>) : go(k_lqr_wave<2, true, 4, fa, as>); break;
+          case 13: waves ? gow(k_lqr_waves<3, true, 1, fa, as>) : go(k_lqr_wave<3, true, 1, fa, as>); break;
+          case 14: waves ? gow(k_lqr_waves<3, true, 2, fa, as>) : go(k_lqr_wave<3, true, 2, fa, as>); break;
+          case 15: waves ? gow(k_lqr_waves<3, true, 3, fa, as>) : go(k_lqr_wave<3, true, 3, fa, as>); break;
+          default: waves ? gow(k_lqr_waves<3, true, 4, fa, as>) : go(k_lqr_wave<3, true, 4, fa, as>); break;
         }
       };
       // n % 4 == 0: the homogeneous offset n alone in the last k step of the
@@ -786,9 +797,9 @@ mpxkkt_status run_lqr_wave(hipStream_t st, const mpxkkt_problem* pr, const Prob<
       else if (as) cases(std::false_type{}, std::true_type{});
       else cases(std::false_type{}, std::false_type{});
     } else {   // stage-varying data: the generic step count (the steps past n + 1 add zeros)
-      if (NT == 1) go(k_lqr_wave<1, false, 4, false, false>);
-      else if (NT == 2) go(k_lqr_wave<2, false, 4, false, false>);
-      else go(k_lqr_wave<3, false, 4, false, false>);
+      if (NT == 1) waves ? gow(k_lqr_waves<1, false, 4, false, false>) : go(k_lqr_wave<1, false, 4, false, false>);
+      else if (NT == 2) waves ? gow(k_lqr_waves<2, false, 4, false, false>) : go(k_lqr_wave<2, false, 4, false, false>);
+      else waves ? gow(k_lqr_waves<3, false, 4, false, false>) : go(k_lqr_wave<3, false, 4, false, false>);
     }
     return launch_check("k_lqr_wave");
   } else {

@@ -651,9 +651,12 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
   return launch_check("k_fwd_stage");
 }
 
-// K1: with flags bit 3 parallel over stages with shared constants
-// (k_linearize_stage: lower latency for small batches) when n, m, n_eq <= 64
-// and its LDS plan fits; else the matrix-core form (k_linearize_mma, 16 stages
+// K1: with flags bit 3, and for the stage-varying model, parallel over stages
+// (k_linearize_stage, the values of k_linearize_inst) when n, m, n_eq <= 64 and
+// its LDS plan fits -- the stage-varying model shares next to nothing between
+// the stages of an instance, so a wave per stage only adds waves in flight (whole
+// iterations at 19 x 7 x 33 p = 3: B = 1 210 -> 163 us, 333 308 -> 269, 1024 525 ->
+// 524; 36 x 12 x 33 B = 333 437 -> 399; FP64 B = 1024 1896 -> 1834); else the matrix-core form (k_linearize_mma, 16 stages
 // per wave, and k_linearize_term) where mma_tiles allows it; else one block
 // per instance (k_linearize_inst, higher throughput for large batches) under
 // the limits of k_linearize_stage; the general block kernel otherwise.
@@ -661,7 +664,8 @@ template <typename T>
 mpxkkt_status run_linearize(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R,
                             const Iter<T>& I, const Ws<T>& W) {
   const bool caller = pr->model == MPXKKT_MODEL_CALLER;
-  if (!caller && (R.flags & 8) != 0 && pr->n <= 64 && pr->m <= 64 && pr->n_eq <= 64) {
+  if (!caller && ((R.flags & 8) != 0 || pr->model == MPXKKT_MODEL_LTV) && pr->n <= 64 && pr->m <= 64 &&
+      pr->n_eq <= 64) {
     const InstLds L = inst_lds(pr->n, pr->m, pr->horizon, pr->model == MPXKKT_MODEL_TANH, pr->Q.stage_stride == 0,
                                pr->R.stage_stride == 0, false);
     const size_t lds =

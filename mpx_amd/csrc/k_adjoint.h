@@ -125,11 +125,13 @@ __device__ __forceinline__ void adj_out(const float (&lam)[NT], const float (&xr
   }
 }
 
+// (a wave per instance, one or kWaveBlock of them per block; the waves never meet)
 template <int NT, bool WIDE>
-__global__ void __launch_bounds__(64) k_adjoint_tanh(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws) {
-  const int b = blockIdx.x;
-  if (skip_instance(ws, b)) return;
-  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+__global__ void __launch_bounds__(64 * kWaveBlock)
+k_adjoint_tanh(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws) {
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x * (blockDim.x >> 6) + wv;
+  if (b >= P.B || skip_instance(ws, b)) return;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;
   const float hs = P.h, hk = P.h * P.kappa, rc = prm.rho_c;
   const AdjR R = adj_rsrc(P, it, ws, b);
@@ -175,7 +177,8 @@ __global__ void __launch_bounds__(64) k_adjoint_tanh(Prob<float> P, Prm<float> p
   // Q (rows 16 i + c, columns 16 k + 4 g + s) in registers; (I + h A)' and
   // (h kappa W)' in the same layout in LDS, each lane reading back only its
   // own entries
-  __shared__ f4 atw[2 * NT * NT * 64];
+  __shared__ f4 atws[kWaveBlock][2 * NT * NT * 64];
+  f4* atw = atws[wv];
   f4 Qt[NT][NT];
   {
     f4 At[NT][NT], Wt[NT][NT];

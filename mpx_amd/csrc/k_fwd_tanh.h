@@ -52,13 +52,16 @@ __device__ __forceinline__ float lane_read(float x, int src) {
 
 // (h kappa W stays in LDS, each lane reading back only its own entries, so
 // that the kernel fits 128 VGPRs: four waves per SIMD, the whole batch of
-// 4096 instances resident at once on 1024 SIMDs)
+// 4096 instances resident at once on 1024 SIMDs; a wave per instance, one or
+// kWaveBlock of them per block, the waves never meet)
 template <int NT, bool WIDE, int R>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WIDE ? 4 : 3))) k_fwd_tanh(Prob<float> P, Ws<float> ws) {
-  __shared__ f4 wl[NT * NT * 64];
-  const int b = blockIdx.x;
-  if (skip_instance(ws, b)) return;
-  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+__global__ void __launch_bounds__(64 * kWaveBlock) __attribute__((amdgpu_waves_per_eu(WIDE ? 4 : 3)))
+k_fwd_tanh(Prob<float> P, Ws<float> ws) {
+  __shared__ f4 wls[kWaveBlock][NT * NT * 64];
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x * (blockDim.x >> 6) + wv;
+  if (b >= P.B || skip_instance(ws, b)) return;
+  f4* wl = wls[wv];
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int n = P.n, m = P.m, N = P.N, N1 = N + 1;
   const float hs = P.h, hk = P.h * P.kappa;
   int off[NT][4];

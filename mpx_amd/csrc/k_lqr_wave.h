@@ -92,15 +92,15 @@ __device__ __forceinline__ float f4_at(const f4& x, int v) {
 
 __device__ __forceinline__ f4 zero4() { return f4{0.f, 0.f, 0.f, 0.f}; }
 
-// Tile transpose through LDS (one wave per block: the barrier is the wave's own).
+// Tile transpose within a wave, through its own buf (16 x 17 floats) in LDS.
 __device__ __forceinline__ f4 tile_transpose(const f4& x, float* buf, int g, int c) {
 #pragma unroll
   for (int v = 0; v < 4; ++v) buf[(4 * g + v) * 17 + c] = x[v];
-  __syncthreads();
+  wave_lds_sync();
   f4 y;
 #pragma unroll
   for (int v = 0; v < 4; ++v) y[v] = buf[c * 17 + 4 * g + v];
-  __syncthreads();
+  wave_lds_sync();
   return y;
 }
 
@@ -478,21 +478,28 @@ __device__ __forceinline__ void il_store_value(const f4 (&S)[NT][NT], const Ws<f
 // and row n's part is added on the vector ALU: column n of S~ A~ gains column
 // n of S~, and row n of A~' (S~ A~) gains row n of S~ A~ (254 instead of 276
 // matrix instructions per stage at n = 36, m = 12, p = 8).
+// A block holds kWaveBlock instances, a wave each, which never meet: the waves
+// of one block sit on different SIMDs.  One-wave blocks were placed by whatever
+// ran before: at 24 x 12 x 100, B = 1024 (a wave per SIMD if spread evenly) the
+// kernel took 348 us behind one predecessor and 508 behind another; this way 350 behind both.
+constexpr int kWaveBlock = 4;
 template <int NT, bool CQ, int KSN, bool FA, bool AS>
-__global__ void __launch_bounds__(64, 2) k_lqr_wave(Prob<float> P, Prm<float> prm, Iter<float> it_unused,
+__global__ void __launch_bounds__(64 * kWaveBlock, 2) k_lqr_wave(Prob<float> P, Prm<float> prm, Iter<float> it_unused,
                                                     Ws<float> ws, LqrIn<float> in) {
   static_assert(!FA || CQ, "A~ is formed from stage-invariant A, W only with stage-invariant Q, B, R");
   static_assert(!AS || CQ, "the homogeneous step is split off only with the step count of n");
   constexpr int KSS = AS ? KSN - 1 : KSN;   // steps of the last state tile in a contraction over the state
   (void)it_unused;
-  const int b = blockIdx.x;
-  if (skip_instance(ws, b)) return;
-  const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x * kWaveBlock + wv;
+  if (b >= P.B || skip_instance(ws, b)) return;
+  const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;
-  __shared__ float tbuf[16 * 17];
+  __shared__ float tbufs[kWaveBlock][16 * 17];
   // FA: the lane's entries of the tiles of I + h A and h kappa W (rows and
   // columns past n - 1 are 0), each lane reading back only its own
-  __shared__ f4 fab[FA ? 2 * NT * NT * 64 : 1];
+  __shared__ f4 fabs_[kWaveBlock][FA ? 2 * NT * NT * 64 : 1];
+  float* tbuf = tbufs[wv];
+  f4* fab = fabs_[wv];
   const float sr = sqrtf(prm.rho_c);
   // k steps over m and over p
   const int ksm = (m + 3) >> 2, ksp = (p + 3) >> 2;

@@ -25,18 +25,6 @@ struct WavesLds {
   float tbuf[NT + 1][16 * 17];
 };
 
-// tile_transpose within a wave of a larger block
-__device__ __forceinline__ f4 wave_transpose(const f4& x, float* buf, int g, int c) {
-#pragma unroll
-  for (int v = 0; v < 4; ++v) buf[(4 * g + v) * 17 + c] = x[v];
-  wave_lds_sync();
-  f4 y;
-#pragma unroll
-  for (int v = 0; v < 4; ++v) y[v] = buf[c * 17 + 4 * g + v];
-  wave_lds_sync();
-  return y;
-}
-
 // Wave J's data of stage t beyond E and r: columns <= J of A~ (FA: sech^2
 // instead, and column n's c), D, q or Q~'s tiles (., J), B~.
 template <int NT, int J, bool CQ, bool FA>
@@ -255,13 +243,13 @@ __device__ __forceinline__ void waves_column(const Prob<float>& P, const Prm<flo
       }
     });
     {
-      const f4 d = wave_transpose(S[J][J], tbuf, g, c);
+      const f4 d = tile_transpose(S[J][J], tbuf, g, c);
 #pragma unroll
       for (int v = 0; v < 4; ++v) S[J][J][v] = 0.5f * (S[J][J][v] + d[v]);
     }
 #pragma unroll
     for (int i = 0; i < J; ++i) {
-      S[J][i] = wave_transpose(S[i][J], tbuf, g, c);
+      S[J][i] = tile_transpose(S[i][J], tbuf, g, c);
       lds.S[J * NT + i][lane] = S[J][i];
       lds.S[i * NT + J][lane] = S[i][J];
     }
@@ -340,7 +328,7 @@ __device__ __forceinline__ void waves_factor(const Prob<float>& P, const Prm<flo
     for (int v = 0; v < 4; ++v) Z[v] = dmask[v];
     with_steps<1, 4>(ksm, [&](auto KM) { chol_lower_inv<decltype(KM)::value>(H, Z, prm.hfloor); });
     lds.Z[lane] = Z;
-    lds.Zt[lane] = wave_transpose(Z, lds.tbuf[NT], g, c);
+    lds.Zt[lane] = tile_transpose(Z, lds.tbuf[NT], g, c);
     lds_sync();
     lds_sync();
     lds_sync();

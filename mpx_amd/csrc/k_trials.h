@@ -6,10 +6,9 @@
 //                boundary steps of the box slacks and multipliers;
 //   k_trials     one wave per stage: that stage's part of phi(a_j) for the
 //                trials a_j = a_max beta^j, j0 <= j < j1;
-//   k_ls_decide  one wave per instance: the first a_j that passes the Armijo
-//                test (the stage parts summed in a fixed order);
-//   k_ls_update  one thread per entry: the multiplier and iterate update at
-//                the accepted step.
+//   k_ls_accept  the first a_j that passes the Armijo test (the stage parts
+//                summed in a fixed order), the multiplier and iterate update
+//                at the accepted step.
 //
 // At a trial point x = X + a dX, u = U + a dU every matrix product of the
 // merit is affine in a: A x = A X + a A dX, W x, B u, Q (x - xr), R (u - ur),
@@ -34,7 +33,7 @@
 
 namespace mpxk {
 
-enum { LS_RHO = 0, LS_PHI0 = 1, LS_DPHI = 2, LS_AMAX = 3, LS_ADUAL = 4, LS_SLACK = 5, LS_ALPHA = 6, NLS = 8 };
+enum { LS_RHO = 0, LS_PHI0 = 1, LS_DPHI = 2, LS_AMAX = 3, LS_ADUAL = 4, LS_SLACK = 5, NLS = 8 };
 constexpr int kTrialWaves = 4;
 
 // Elements of one wave's LDS vectors in k_trials: x0 = X_t, x1 = dX_t,
@@ -414,92 +413,102 @@ __global__ void __launch_bounds__(512) k_trials(Prob<T> P, Prm<T> prm, Iter<T> i
   }
 }
 
-// The accepted step of instance blockIdx.x (one wave): the first trial that
-// passes the Armijo test, else the last one (status 2); the trial count
-// reported is that of backtracking in groups of prm.group.  Writes the step
-// to lsp[LS_ALPHA] for k_ls_update and the instance's report.
-template <typename T>
-__global__ void __launch_bounds__(64) k_ls_decide(Prm<T> prm, Ws<T> ws, int N1, T* o_alpha, T* o_rho, T* o_phi0,
-                                                  T* o_dphi, int* o_status, int* o_trials) {
-  const int b = blockIdx.x, lane = threadIdx.x;
-  if (skip_instance(ws, b)) return;
-  T* ls = ws.lsp + (size_t)b * NLS;
-  const int MT = prm.max_trials, g = prm.group;
-  const int js = ls_first_accept(prm, ws, b, N1, MT);
-  T alpha = ls[LS_AMAX];
-  int status = 0, trials = MT;
-  if (js >= 0) {
-    for (int q = 0; q < js; ++q) alpha *= prm.beta;
-    trials = (js / g + 1) * g;
-    trials = trials < MT ? trials : MT;
-  } else {
-    for (int q = 0; q < MT - 1; ++q) alpha *= prm.beta;
-    status = 2;
-  }
-  const T rho = ls[LS_RHO], phi0 = ls[LS_PHI0], dphi = ls[LS_DPHI];
-  if (!isfinite(phi0) || !isfinite(dphi)) status = 1;
-  if (lane == 0) {
-    ls[LS_ALPHA] = alpha;
-    if (o_alpha) o_alpha[b] = alpha;
-    if (o_rho) o_rho[b] = rho;
-    if (o_phi0) o_phi0[b] = phi0;
-    if (o_dphi) o_dphi[b] = dphi;
-    if (o_status) o_status[b] = status;
-    if (o_trials) o_trials[b] = trials;
-  }
-}
+// The acceptance of instance blockIdx.y: the step a (the first trial that passes
+// the Armijo test, else the last one: status 2; the trial count reported is that
+// of backtracking in groups of prm.group), then the iterate and multipliers at
+// it, in parts of kAcceptEntries per thread: parts [0, nbx) X += a dX and V += a
+// dV, the next nbu U += a dU with the box multipliers' update (at u before the
+// step), the rest Y_eq += rho_c (h + a dh) from the equality rows and slopes the
+// trials stored.  Every block finds the step itself, from the merit parts; block
+// 0 reports it.  A kernel for the step and one for the update took 9 us of a
+// single problem's iteration, this one 5.
+constexpr int kAcceptEntries = 4;
 
-// Iterate and multiplier update at the accepted step a = lsp[LS_ALPHA], one
-// thread per entry: blocks [0, nbx) take X += a dX and V += a dV, the next
-// nbu blocks U += a dU with the box multipliers' update (at u before the
-// step), the rest Y_eq += rho_c (h + a dh) from the equality rows and slopes
-// the trials stored.
 template <typename T>
-__global__ void __launch_bounds__(256) k_ls_update(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws, int nbx, int nbu) {
-  const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;
-  const size_t B = (size_t)P.B;
-  int blk = blockIdx.x;
-  if (blk < nbx) {
-    const size_t e = (size_t)blk * 256 + threadIdx.x;
-    if (e >= B * N1 * n) return;
-    const int b = (int)(e / ((size_t)N1 * n));
-    if (skip_instance(ws, b)) return;
-    const T a = ws.lsp[(size_t)b * NLS + LS_ALPHA];
-    it.X[e] += a * ws.dx[e];
-    it.V[e] += a * ws.dv[e];
-    return;
-  }
-  blk -= nbx;
-  if (blk < nbu) {
-    const size_t e = (size_t)blk * 256 + threadIdx.x;
-    if (e >= B * N * m) return;
-    const int b = (int)(e / ((size_t)N * m));
-    if (skip_instance(ws, b)) return;
-    const int r = (int)(e - (size_t)b * N * m), t = r / m, i = r - t * m;
-    const T* ls = ws.lsp + (size_t)b * NLS;
-    const T a = ls[LS_ALPHA];
-    const T u = it.U[e], du = ws.du[e];
-    if (P.box) {
-      const T adual = ls[LS_ADUAL];
-      const T lo = P.ulo.at(b, t)[i], hi = P.uhi.at(b, t)[i];
-      const T shi = hi - u, slo = u - lo;
-      T* nu = it.Ybox + ((size_t)b * N + t) * 2 * m;
-      const T nhi = nu[i], nlo = nu[m + i];
-      nu[i] = nhi + adual * (prm.mu_b / shi - nhi + nhi * du / shi);
-      nu[m + i] = nlo + adual * (prm.mu_b / slo - nlo - nlo * du / slo);
-    }
-    it.U[e] = u + a * du;
-    return;
-  }
-  blk -= nbu;
-  const size_t e = (size_t)blk * 256 + threadIdx.x;
-  if (p == 0 || e >= B * N * p) return;
-  const int b = (int)(e / ((size_t)N * p));
+__global__ void __launch_bounds__(256) k_ls_accept(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws, int nbx, int nbu,
+                                                   int nparts, T* o_alpha, T* o_rho, T* o_phi0, T* o_dphi, int* o_status,
+                                                   int* o_trials) {
+  const int b = blockIdx.y, tid = threadIdx.x;
   if (skip_instance(ws, b)) return;
-  const int r = (int)(e - (size_t)b * N * p), t = r / p, k = r - t * p;
-  const T a = ws.lsp[(size_t)b * NLS + LS_ALPHA];
-  const T* hq = ws.hq + ((size_t)b * N + t) * 2 * p;
-  it.Yeq[e] += prm.rho_c * (hq[k] + a * hq[p + k]);
+  const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;
+  const T* ls = ws.lsp + (size_t)b * NLS;
+  __shared__ T step;
+  if (tid < 64) {
+    const int MT = prm.max_trials, g = prm.group;
+    const int js = ls_first_accept(prm, ws, b, N1, MT);
+    T alpha = ls[LS_AMAX];
+    int status = 0, trials = MT;
+    if (js >= 0) {
+      for (int q = 0; q < js; ++q) alpha *= prm.beta;
+      trials = (js / g + 1) * g;
+      trials = trials < MT ? trials : MT;
+    } else {
+      for (int q = 0; q < MT - 1; ++q) alpha *= prm.beta;
+      status = 2;
+    }
+    if (tid == 0) {
+      step = alpha;
+      if (blockIdx.x == 0) {
+        const T rho = ls[LS_RHO], phi0 = ls[LS_PHI0], dphi = ls[LS_DPHI];
+        if (!isfinite(phi0) || !isfinite(dphi)) status = 1;
+        if (o_alpha) o_alpha[b] = alpha;
+        if (o_rho) o_rho[b] = rho;
+        if (o_phi0) o_phi0[b] = phi0;
+        if (o_dphi) o_dphi[b] = dphi;
+        if (o_status) o_status[b] = status;
+        if (o_trials) o_trials[b] = trials;
+      }
+    }
+  }
+  __syncthreads();
+  const T a = step, adual = ls[LS_ADUAL];
+  for (int part = blockIdx.x; part < nparts; part += gridDim.x) {
+    int blk = part;
+    if (blk < nbx) {
+      const size_t o = (size_t)b * N1 * n;
+#pragma unroll
+      for (int k = 0; k < kAcceptEntries; ++k) {
+        const int e = (blk * kAcceptEntries + k) * 256 + tid;
+        if (e < N1 * n) {
+          it.X[o + e] += a * ws.dx[o + e];
+          it.V[o + e] += a * ws.dv[o + e];
+        }
+      }
+      continue;
+    }
+    blk -= nbx;
+    if (blk < nbu) {
+#pragma unroll
+      for (int k = 0; k < kAcceptEntries; ++k) {
+        const int r = (blk * kAcceptEntries + k) * 256 + tid;
+        if (r < N * m) {
+          const size_t e = (size_t)b * N * m + r;
+          const T u = it.U[e], du = ws.du[e];
+          if (P.box) {
+            const int t = r / m, i = r - t * m;
+            const T lo = P.ulo.at(b, t)[i], hi = P.uhi.at(b, t)[i];
+            const T shi = hi - u, slo = u - lo;
+            T* nu = it.Ybox + ((size_t)b * N + t) * 2 * m;
+            const T nhi = nu[i], nlo = nu[m + i];
+            nu[i] = nhi + adual * (prm.mu_b / shi - nhi + nhi * du / shi);
+            nu[m + i] = nlo + adual * (prm.mu_b / slo - nlo - nlo * du / slo);
+          }
+          it.U[e] = u + a * du;
+        }
+      }
+      continue;
+    }
+    blk -= nbu;
+#pragma unroll
+    for (int k = 0; k < kAcceptEntries; ++k) {
+      const int r = (blk * kAcceptEntries + k) * 256 + tid;
+      if (r < N * p) {
+        const int t = r / p, q = r - t * p;
+        const T* hq = ws.hq + ((size_t)b * N + t) * 2 * p;
+        it.Yeq[(size_t)b * N * p + r] += prm.rho_c * (hq[q] + a * hq[p + q]);
+      }
+    }
+  }
 }
 
 }  // namespace mpxk

@@ -575,6 +575,14 @@ bool fx_in_lqr(const mpxkkt_problem* pr, const Prm<T>& R) {
   return use_wave_lqr<T>(pr, R) && (R.flags & 8) == 0 && mma_tiles<T>(pr, R.flags) > 0;
 }
 
+// Up to this many instances the wave recursion takes NT + 1 waves per instance
+// (k_lqr_waves, the same bits), past it one: with 1024 SIMDs the extra waves are
+// free until each has one, then the one-wave form's fewer instructions win.
+// Iterations at 36 x 12 x 50 p = 8, one wave -> NT + 1: B = 1 453 -> 301 us, 256
+// 481 -> 332, 512 508 -> 420, 768 549 -> 608; 45 x 14 x 50 B = 512 648 -> 599, 768
+// 709 -> 827; 24 x 12 x 50 B = 512 315 -> 282, 1024 351 -> 425.
+constexpr int kWavesBatch = 512;
+
 // costates, control steps and slope partials: on the wave path the forward
 // pass of the LQR solve and the costates -- for the tanh model after
 // k_linearize_mma k_fwd_tanh and the adjoint sweep k_adjoint_tanh, else
@@ -593,7 +601,11 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
       const int nf = fx_in_lqr<T>(pr, R) ? mma_tiles<T>(pr, R.flags) : 0;
       if (nf) {
         const bool wide = mma_rows16<T>(pr) && al16(W.K) && al16(W.cdef) && al16(W.dx);
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, st, P, W); };
+        // one wave per block where every instance has a CU's SIMD to itself
+        // anyway, else blocks whose waves sit on different SIMDs (kWaveBlock)
+        const int wpb = pr->batch <= kWavesBatch ? 1 : kWaveBlock;
+        const dim3 gw((pr->batch + wpb - 1) / wpb), bw(64 * wpb);
+        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, gw, bw, 0, st, P, W); };
         if (wide) {
           if (nf == 1) go(k_fwd_tanh<1, true, 4>);
           else if (nf == 2) go(k_fwd_tanh<2, true, 4>);
@@ -606,7 +618,7 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
         mpxkkt_status s = launch_check("k_fwd_tanh");
         if (s != MPXKKT_OK) return s;
         // the costates by the adjoint recursion (k_lqr_wave stored no S_t)
-        auto goa = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, st, P, R, I, W); };
+        auto goa = [&](auto kern) { hipLaunchKernelGGL(kern, gw, bw, 0, st, P, R, I, W); };
         if (wide) {
           if (nf == 1) goa(k_adjoint_tanh<1, true>);
           else if (nf == 2) goa(k_adjoint_tanh<2, true>);
@@ -657,7 +669,7 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
 // the stages of an instance, so a wave per stage only adds waves in flight (whole
 // iterations at 19 x 7 x 33 p = 3: B = 1 210 -> 163 us, 333 308 -> 269, 1024 525 ->
 // 524; 36 x 12 x 33 B = 333 437 -> 399; FP64 B = 1024 1896 -> 1834); else the matrix-core form (k_linearize_mma, 16 stages
-// per wave, and k_linearize_term) where mma_tiles allows it; else one block
+// per wave) where mma_tiles allows it; else one block
 // per instance (k_linearize_inst, higher throughput for large batches) under
 // the limits of k_linearize_stage; the general block kernel otherwise.
 template <typename T>
@@ -686,7 +698,7 @@ mpxkkt_status run_linearize(hipStream_t st, const mpxkkt_problem* pr, const Prob
       const bool wide = mma_rows16<T>(pr) && al16(I.X) && al16(I.U) && al16(I.V) &&
                         (!pr->has_box || al16(I.Ybox)) && al16(W.qh) && al16(W.cdef) && al16(W.rh) &&
                         al16(W.rd) && al16(W.Alin) && al16(W.sdh);
-      const dim3 grid((pr->horizon + 15) / 16, pr->batch);
+      const dim3 grid((pr->horizon + 15) / 16 + 1, pr->batch);
       // f_x only for the LQR kernels that read it
       const int wfx = fx_in_lqr<T>(pr, R) ? 0 : 1;
       auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(64), 0, st, P, R, I, W, wfx); };
@@ -699,19 +711,7 @@ mpxkkt_status run_linearize(hipStream_t st, const mpxkkt_problem* pr, const Prob
         else if (nt == 2) go(k_linearize_mma<2, false>);
         else go(k_linearize_mma<3, false>);
       }
-      mpxkkt_status s = launch_check("k_linearize_mma");
-      if (s != MPXKKT_OK) return s;
-      auto got = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(pr->batch), dim3(64), 0, st, P, I, W); };
-      if (wide) {
-        if (nt == 1) got(k_linearize_term<1, true>);
-        else if (nt == 2) got(k_linearize_term<2, true>);
-        else got(k_linearize_term<3, true>);
-      } else {
-        if (nt == 1) got(k_linearize_term<1, false>);
-        else if (nt == 2) got(k_linearize_term<2, false>);
-        else got(k_linearize_term<3, false>);
-      }
-      return launch_check("k_linearize_term");
+      return launch_check("k_linearize_mma");
     }
   }
   if (const int rt = caller ? 0 : rows_tiles<T>(pr, R.flags)) {
@@ -752,14 +752,6 @@ bool use_wave_lqr(const mpxkkt_problem* pr, const Prm<T>& R) {
   return IsF32<T>::value && wave_path(pr, R.flags, R.P);
 }
 
-// Up to this many instances the wave recursion takes NT + 1 waves per instance
-// (k_lqr_waves, the same bits), past it one: with 1024 SIMDs the extra waves are
-// free until each has one, then the one-wave form's fewer instructions win.
-// Iterations at 36 x 12 x 50 p = 8, one wave -> NT + 1: B = 1 453 -> 301 us, 256
-// 481 -> 332, 512 508 -> 420, 768 549 -> 608; 45 x 14 x 50 B = 512 648 -> 599, 768
-// 709 -> 827; 24 x 12 x 50 B = 512 315 -> 282, 1024 351 -> 425.
-constexpr int kWavesBatch = 512;
-
 template <typename T>
 mpxkkt_status run_lqr_wave(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R,
                            const Iter<T>& I, const Ws<T>& W, const LqrIn<T>& in) {
@@ -769,7 +761,10 @@ mpxkkt_status run_lqr_wave(hipStream_t st, const mpxkkt_problem* pr, const Prob<
     const int ksn = (pr->n + 1 - 16 * (NT - 1) + 3) / 4;
     const bool cq = P.Q.st == 0 && P.R.st == 0 && in.Bm.st == 0;   // Q, B, R held for the whole recursion
     const dim3 gb(pr->batch);
-    auto go = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64), 0, st, P, R, I, W, in); };
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, dim3((pr->batch + kWaveBlock - 1) / kWaveBlock), dim3(64 * kWaveBlock), 0, st, P, R, I, W,
+                         in);
+    };
     auto gow = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64 * (NT + 1)), 0, st, P, R, W, in); };
     const bool waves = pr->batch <= kWavesBatch;
     if (cq) {
@@ -950,29 +945,32 @@ mpxkkt_status run_trials(hipStream_t st, const mpxkkt_problem* pr, const TrialSh
   return launch_trials<T, 8>(st, ts, P, R, I, W, j0, j1);
 }
 
-// The acceptance: k_ls_decide (the step, once per instance), then k_ls_update
-// (the iterate and multipliers, one thread per entry).
+// The acceptance: k_ls_accept (the step, the iterate and the multipliers).
+constexpr int kAcceptBlocks = 2048;   // eight per CU
+
 template <typename T>
 mpxkkt_status ls_accept(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R,
                         const Iter<T>& I, const Ws<T>& W, const mpxkkt_stats* so) {
-  const size_t B = pr->batch, n = pr->n, m = pr->m, p = pr->n_eq, N = pr->horizon, N1 = N + 1;
+  const int n = pr->n, m = pr->m, p = pr->n_eq, N = pr->horizon, N1 = N + 1;
   T* a = so ? static_cast<T*>(so->alpha) : nullptr;
   T* r = so ? static_cast<T*>(so->rho) : nullptr;
   T* f0 = so ? static_cast<T*>(so->merit0) : nullptr;
   T* df = so ? static_cast<T*>(so->dmerit) : nullptr;
   int* stt = so ? so->status : nullptr;
   int* tr = so ? so->trials : nullptr;
-  hipLaunchKernelGGL(k_ls_decide<T>, dim3((unsigned)B), dim3(64), 0, st, R, W, (int)N1, a, r, f0, df, stt, tr);
-  mpxkkt_status s = launch_check("k_ls_decide");
-  if (s != MPXKKT_OK) return s;
-  const int nbx = (int)((B * N1 * n + 255) / 256), nbu = (int)((B * N * m + 255) / 256);
-  const int nbp = (int)((B * N * p + 255) / 256);
-  hipLaunchKernelGGL(k_ls_update<T>, dim3(nbx + nbu + nbp), dim3(256), 0, st, P, R, I, W, nbx, nbu);
-  return launch_check("k_ls_update");
+  const int per = kAcceptEntries * 256, nbx = (N1 * n + per - 1) / per, nbu = (N * m + per - 1) / per;
+  const int nbp = (N * p + per - 1) / per, parts = nbx + nbu + nbp;
+  // a block per part for few instances; for many one per instance, which finds
+  // the step once (36 x 12 x 50 p = 8, B = 4096: 42 us, a block per part 65, a
+  // kernel of its own for the step 47)
+  const int blocks = std::min(parts, std::max(1, kAcceptBlocks / pr->batch));
+  hipLaunchKernelGGL(k_ls_accept<T>, dim3(blocks, pr->batch), dim3(256), 0, st, P, R, I, W, nbx, nbu, parts, a, r, f0, df,
+                     stt, tr);
+  return launch_check("k_ls_accept");
 }
 
 // K4: k_ls_setup, k_trials over [0, group) and then [group, max_trials) for the
-// instances that accepted none of the first group, k_ls_decide and k_ls_update.  flags bit 2
+// instances that accepted none of the first group, k_ls_accept.  flags bit 2
 // selects the single-kernel line search of k_inst.h / k_linesearch.h instead.
 template <typename T>
 mpxkkt_status run_linesearch(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R,

@@ -198,7 +198,7 @@ __device__ __forceinline__ int tile_upper(int u) {
   return u - j * (j + 1) / 2 + 16 * j;
 }
 
-enum { TILE_A = 0, TILE_FX = 1, TILE_CALLER = 2 };
+enum { TILE_A = 0, TILE_CALLER = 1 };
 
 // FP32: Z = L^{-1} of the floored Cholesky factor of H (16 MT square, identity
 // past m), in two halves, from its upper tiles in the registers of one wave, to
@@ -322,9 +322,8 @@ struct TileFactor<double, 1> {
 };
 
 // n + 1 <= 16 NT (NT minimal), 16 (MT - 1) < m <= 16 MT, p <= 16.  Stores K~_t
-// and, with store_s, the upper tiles of S_t and s_t (k_costate_rows).  MODE:
-// TILE_FX forms f_x = I + h (A + kappa diag(sd_t) W) of the tanh model from
-// sd_t = ws.sdh; TILE_CALLER adds the caller's cross Hessian M_t (may be null).
+// and, with store_s, the upper tiles of S_t and s_t (k_costate_rows).  MODE
+// TILE_CALLER adds the caller's cross Hessian M_t (may be null).
 // FP64: m <= 16, n + 1 <= 64, both triangles of S_t.
 template <typename T, int NT, int MT, int NW, int MODE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
@@ -362,7 +361,6 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
   const long long sA = in.A.st, sB = in.Bm.st, sQ = P.Q.st, sR = P.R.st, sD = P.D.st, sE = P.E.st, sM = P.M.st;
   const T *pc_ = ws.cdef + ((size_t)b * N1 + 1) * n, *pq = ws.qh + (size_t)b * N1 * n;
   const T *pr = ws.rh + (size_t)b * N * m, *prd = ws.rd + (size_t)b * N * m;
-  const T* psd = ws.sdh + (size_t)b * N * n;
   T *pK = ws.K + (size_t)b * N * m * n, *pk = ws.k + (size_t)b * N * m;
   T *pS = ws.S + (size_t)b * N1 * n * n, *ps = ws.s + (size_t)b * N1 * n;
 
@@ -395,9 +393,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
                  : role == 1 ? block_of(ts, 1, na, n, X::DT, LP)
                              : block_of(role == 2 ? ts : -1, 1, mb, m, X::ET, LP);
   V4 ra[4], rb[4], rcv;
-  V4 fa[MODE == TILE_FX ? 4 : 1], fw[MODE == TILE_FX ? 4 : 1];
   T rvr, rvd, rvq, rdg;
-  const int sdo = (16 * ((tid >> 4) / na) + ((tid >> 2) & 3)) * ES;   // sd_t of a block's first row
   // (absent entries past the descriptor: branches around loads would make the
   // later waits, which count requests, wait for more than they need)
   const int cvo = tid < 4 * NT ? (16 * (tid >> 2) + (tid & 3)) * ES : kOOB;
@@ -421,15 +417,9 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
       const int cols = role == 1 ? n : m, rows = role == 0 ? n : p;
       block_load(rb, tile_rsrc(q, rows * cols), kb.off, cols);
     }
-    if constexpr (MODE == TILE_FX) {
-      const rsrc_t rs = tile_rsrc(psd + (size_t)t * n, n);
-#pragma unroll
-      for (int s = 0; s < 4; ++s) ra[0][s] = O::bload(rs, sdo, 4 * s * ES);
-    } else {
-      const rsrc_t rA = tile_rsrc(pA + t * sA, n * n);
-      block_load(ra, rA, ka.off, n);
-      rdg = O::bload(rA, dgo);
-    }
+    const rsrc_t rA = tile_rsrc(pA + t * sA, n * n);
+    block_load(ra, rA, ka.off, n);
+    rdg = O::bload(rA, dgo);
     const rsrc_t rc = tile_rsrc(pc_ + (size_t)t * n, n);
 #pragma unroll
     for (int s = 0; s < 4; ++s) rcv[s] = O::bload(rc, cvo, 4 * s * ES);
@@ -438,16 +428,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
     rvq = O::bload(tile_rsrc(pq + (size_t)t * n, n), qvo);
   };
   auto store_data = [&]() {
-    if constexpr (MODE == TILE_FX) {   // f_x - I by rows: h A + sd h kappa W
-      V4 x[4];
-#pragma unroll
-      for (int s = 0; s < 4; ++s)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) x[s][j] = fa[s][j] + ra[0][s] * fw[s][j];
-      block_store(x, ka);
-    } else {
-      block_store(ra, ka);
-    }
+    block_store(ra, ka);
     if (role == 0 ? !bconst : role < 3 && p > 0) {
       if (role > 0) {
 #pragma unroll
@@ -464,7 +445,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
   };
   // after store_data and a barrier: the unit diagonal taken out of A~
   auto store_diag = [&]() {
-    if (MODE != TILE_FX && tid < n) {
+    if (tid < n) {
       const T e = rdg >= T(0.5) && rdg <= T(2) ? T(1) : T0;
       const int d = tile_pos(tid);
       sm[X::AT + d * LD + d] = rdg - e;
@@ -522,7 +503,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
   // ---- start: LDS cleared (padding rows and columns stay 0), S~_N, stage N - 1
   for (int e = tid; e < X::TOTAL; e += NTH) sm[e] = T0;
   __syncthreads();
-  if (tid < 16 * NT && (tid == pn || (MODE == TILE_FX && tile_pos(tid) < n))) sm[X::EV + tid] = T(1);
+  if (tid < 16 * NT && tid == pn) sm[X::EV + tid] = T(1);
   {
     const T* QN = P.QN.at(b, 0);
     const T* qN = pq + (size_t)N * n;
@@ -536,15 +517,6 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
       sm[X::S + tile_pos(i) * LD + pn] = q;
       sm[X::S + pn * LD + tile_pos(i)] = q;
       if (store_s) ps[(size_t)N * n + i] = q;
-    }
-  }
-  if constexpr (MODE == TILE_FX) {
-    block_load(fa, tile_rsrc(P.A.at(b, 0), n * n), ka.off, n);
-    block_load(fw, tile_rsrc(P.W.at(b, 0), n * n), ka.off, n);
-#pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      fa[s] *= P.h;
-      fw[s] *= P.h * P.kappa;
     }
   }
   if (bconst && role == 0) {

@@ -191,14 +191,13 @@ __device__ int ls_first_accept(const Prm<T>& prm, const Ws<T>& ws, int b, int N1
   return -1;
 }
 
-// Trials j0 <= j < j1 at stage t = t0 + blockIdx.x * waves + wave of instance
+// Trials j0 <= j < j1 at stage t = blockIdx.x * waves + wave of instance
 // blockIdx.y.  RPL: state (and equality) rows per lane, ceil(max(n, p) / 64).
 template <typename T, int RPL, bool V4, bool SH>
-__global__ void __launch_bounds__(512) k_trials(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws, int j0, int j1,
-                                                int t0) {
+__global__ void __launch_bounds__(512) k_trials(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws, int j0, int j1) {
   static_assert(!V4 || IsF32<T>::value, "float4 rows are FP32 only");
   const int wpb = blockDim.x >> 6, wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int b = blockIdx.y, t = t0 + blockIdx.x * wpb + wv;
+  const int b = blockIdx.y, t = blockIdx.x * wpb + wv;
   if (skip_instance(ws, b)) return;
   const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;
   // an earlier pass accepted: the same answer in every wave of the block (one instance)
@@ -411,6 +410,58 @@ __global__ void __launch_bounds__(512) k_trials(Prob<T> P, Prm<T> prm, Iter<T> i
       tp[2 * j + 1] = s2;
     }
   }
+}
+
+// k_trials at the terminal stage alone, by one wave (n <= 64; x1, d0: n entries
+// of LDS each, rounded up to 4): the same sums in the same order.
+template <typename T>
+__device__ __forceinline__ void trial_term(const Prob<T>& P, const Prm<T>& prm, const Iter<T>& it, const Ws<T>& ws,
+                                           int b, int j0, int j1, T* x1, T* d0) {
+  const int lane = threadIdx.x & 63, n = P.n, N = P.N, N1 = N + 1;
+  const size_t oN = ((size_t)b * N1 + N) * n + lane, o0 = (size_t)b * N1 * n + lane;
+  const bool on = lane < n;
+  T dd0 = 0, dd1 = 0, F0 = 0, xn0 = 0, xn1 = 0, vn0 = 0, vn1 = 0, q0 = 0, q1 = 0;
+  if (on) {
+    dd0 = it.X[oN] - P.xref.at(b, N)[lane];
+    dd1 = ws.dx[oN];
+    F0 = P.x0.at(b, 0)[lane];
+    xn0 = it.X[o0];
+    xn1 = ws.dx[o0];
+    vn0 = it.V[o0];
+    vn1 = ws.dv[o0];
+    d0[lane] = dd0;
+    x1[lane] = dd1;
+  }
+  wave_lds_sync();
+  if (on) row_dot2<T, false>(P.QN.at(b, 0) + (size_t)lane * n, n, d0, x1, q0, q1);
+  T a = ws.lsp[(size_t)b * NLS + LS_AMAX];
+  for (int q = 0; q < j0; ++q) a *= prm.beta;
+  T* tp = ws.tpart + ((size_t)b * N1 + N) * 2 * MAX_TRIALS;
+  for (int j = j0; j < j1; ++j, a *= prm.beta) {
+    T s1 = 0, s2 = 0;
+    if (on) {
+      const T F1 = 0, f = F0 + a * F1;
+      const T c = f - (xn0 + a * xn1);
+      const T v = vn0 + a * vn1;
+      s1 += v * c + T(0.5) * (dd0 + a * dd1) * (q0 + a * q1);
+      s2 += c * c;
+    }
+    s1 = wave_sum(s1);
+    s2 = wave_sum(s2);
+    if (lane == 0) {
+      tp[2 * j] = s1;
+      tp[2 * j + 1] = s2;
+    }
+  }
+}
+
+template <typename T>
+__global__ void __launch_bounds__(64) k_trials_term(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws, int j0, int j1) {
+  __shared__ T x1[64], d0[64];
+  const int b = blockIdx.x;
+  if (skip_instance(ws, b)) return;
+  if (j0 > 0 && ls_first_accept(prm, ws, b, P.N + 1, j0) >= 0) return;
+  trial_term<T>(P, prm, it, ws, b, j0, j1, x1, d0);
 }
 
 // The acceptance of instance blockIdx.y: the step a (the first trial that passes

@@ -1,8 +1,7 @@
 // The trial kernel of the line search on the matrix cores, for the tanh model
 // with stage-invariant A, W, B, Q, R (FP32, n <= 48, m <= 16, p <= 16): one
 // wave takes 16 consecutive stages t < N of one instance, stage 16 blockIdx.x +
-// c in lane column c.  The merit parts of k_trials (k_trials.h; the terminal
-// stage stays there) need, per stage, the products of A, W, Q, B and R with the
+// c in lane column c.  The merit parts of k_trials (k_trials.h) need, per stage, the products of A, W, Q, B and R with the
 // stage's vectors at the iterate and along the step; here they are products of
 // the stage-invariant matrices with 16 stages at once: the vectors of the
 // wave's stages are the columns of B-operand tiles (lane (g, c), register v
@@ -97,7 +96,7 @@ __device__ __forceinline__ f4 lds_aop(const float* sm, int i, int k, int g, int 
 }
 
 // Trials j0 <= j < j1 at the stages 64 blockIdx.x + 16 w + c < N of instance
-// blockIdx.y (wave w of the block).  The block stages A, W, Q, B, R in LDS
+// blockIdx.y (wave w of the block); a block past them, where the grid has one, takes the terminal stage.  The block stages A, W, Q, B, R in LDS
 // once (MmaLds); each wave reads its A-operand tiles from there where a
 // product uses them.
 // HQ: the equality rows at the iterate and their slope along the step are
@@ -113,6 +112,10 @@ k_trials_mma(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws, int j0
   const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;
   // an earlier pass accepted: the same answer in every wave (one instance)
   if (j0 > 0 && ls_first_accept(prm, ws, b, N1, j0) >= 0) return;
+  if ((int)blockIdx.x * 64 >= N) {   // a block past the stages: the terminal stage
+    if (wv == 0) trial_term<float>(P, prm, it, ws, b, j0, j1, smA, smW);
+    return;
+  }
   lds_stage<L::ROWS, L::LD>(smA, P.A.at(b, 0), n, n, tid);
   lds_stage<L::ROWS, L::LD>(smW, P.W.at(b, 0), n, n, tid);
   lds_stage<L::ROWS, L::LD>(smQ, P.Q.at(b, 0), n, n, tid);

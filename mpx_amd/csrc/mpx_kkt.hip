@@ -878,9 +878,12 @@ mpxkkt_status launch_trials_k(hipStream_t st, const TrialShape& ts, const Prob<T
   mpxkkt_status s;
   if constexpr (IsF32<T>::value) {
     if (ts.mma) {
-      // stages 0 .. N - 1 on the matrix cores, the terminal stage by one wave of k_trials
+      // stages 0 .. N - 1 on the matrix cores; the terminal stage by one wave of one more block,
+      // for large batches by a launch of its own (36 x 12 x 50: B = 1 296 -> 292 us in the same
+      // launch, B = 4096 1688 -> 1769: its blocks hold the others' LDS)
+      const bool term = P.B <= kWavesBatch;
       const int N = P.N;
-      const dim3 grid((N + 63) / 64, P.B);
+      const dim3 grid((N + 63) / 64 + (term ? 1 : 0), P.B);
       // 128-bit loads when the iterate and the step are 16-byte aligned too
       const bool wide = ts.mma_wide && al16(I.X) && al16(I.U) && al16(I.V) && al16(W.dx) && al16(W.du) &&
                         al16(W.dv);
@@ -900,15 +903,13 @@ mpxkkt_status launch_trials_k(hipStream_t st, const TrialShape& ts, const Prob<T
       // after k_linearize_mma and k_adjoint_tanh the equality rows are in hq
       if (ts.hq) forms(std::true_type{});
       else forms(std::false_type{});
-      if ((s = launch_check("k_trials_mma")) != MPXKKT_OK) return s;
-      const size_t lds = (size_t)trial_wave_elems(P.n, P.m) * sizeof(T);
-      if ((s = prep_lds(k_trials<T, RPL, V4, false>, lds)) != MPXKKT_OK) return s;
-      hipLaunchKernelGGL((k_trials<T, RPL, V4, false>), dim3(1, P.B), dim3(64), lds, st, P, R, I, W, j0, j1, N);
-      return launch_check("k_trials");
+      if ((s = launch_check("k_trials_mma")) != MPXKKT_OK || term) return s;
+      hipLaunchKernelGGL(k_trials_term<T>, dim3(P.B), dim3(64), 0, st, P, R, I, W, j0, j1);
+      return launch_check("k_trials_term");
     }
   }
   if ((s = prep_lds(k_trials<T, RPL, V4, SH>, ts.lds)) != MPXKKT_OK) return s;
-  hipLaunchKernelGGL((k_trials<T, RPL, V4, SH>), ts.grid, dim3(64 * ts.waves), ts.lds, st, P, R, I, W, j0, j1, 0);
+  hipLaunchKernelGGL((k_trials<T, RPL, V4, SH>), ts.grid, dim3(64 * ts.waves), ts.lds, st, P, R, I, W, j0, j1);
   return launch_check("k_trials");
 }
 

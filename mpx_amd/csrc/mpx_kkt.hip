@@ -497,11 +497,20 @@ bool trial_rows16(const mpxkkt_problem* pr) {
   }
 }
 
-// The matrix-core forms of the linearisation and of the trials
-// (k_lin_mma.h, k_trials_mma.h): FP32, the tanh model with stage-invariant A,
-// W, B, Q, R, at most three state tiles, one control tile and one tile of
-// equality rows, and flags bit 4 clear (bit 4 keeps the row-per-lane forms,
-// for comparison).  Returns the number of state tiles, 0 when they do not apply.
+// The FP32 stages 0 .. nst - 1 of a view (len entries each) lie below byte kOOB
+// of one buffer descriptor: 32-bit byte offsets reach every entry and kOOB none.
+bool in_descriptor(const mpxkkt_view& v, long long nst, long long len) {
+  return v.ptr == nullptr || nst < 2 || v.stage_stride <= (kOOB / 4 - len) / (nst - 1);
+}
+
+// The matrix-core forms of the linearisation, of the trials, of the adjoint
+// sweep and of the evaluation (k_lin_mma.h, k_trials_mma.h, k_adjoint.h,
+// k_eval_mma.h): FP32, the tanh model with stage-invariant A, W, B, Q, R, at
+// most three state tiles, one control tile and one tile of equality rows, the
+// other views' whole horizon within one descriptor (a stage-major array of many
+// instances can span more: 4096 x 608 stages of 12 x 36 rows pass 4 GiB), and
+// flags bit 4 clear (bit 4 keeps the row-per-lane forms, for comparison).
+// Returns the number of state tiles, 0 when they do not apply.
 template <typename T>
 int mma_tiles(const mpxkkt_problem* pr, int flags) {
   if (!IsF32<T>::value || pr->model != MPXKKT_MODEL_TANH || (flags & 16) != 0) return 0;
@@ -509,6 +518,11 @@ int mma_tiles(const mpxkkt_problem* pr, int flags) {
       pr->R.stage_stride != 0)
     return 0;
   if (pr->n > 48 || pr->m > 16 || pr->n_eq > 16) return 0;
+  const long long N = pr->horizon, n = pr->n, m = pr->m, p = pr->n_eq;
+  if (!in_descriptor(pr->xref, N + 1, n) || !in_descriptor(pr->uref, N, m)) return 0;
+  if (p > 0 && !(in_descriptor(pr->D, N, p * n) && in_descriptor(pr->E, N, p * m) && in_descriptor(pr->e, N, p)))
+    return 0;
+  if (pr->has_box && !(in_descriptor(pr->ulo, N, m) && in_descriptor(pr->uhi, N, m))) return 0;
   return (pr->n + 15) / 16;
 }
 

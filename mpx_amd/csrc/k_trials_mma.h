@@ -279,7 +279,8 @@ k_trials_mma(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws, int j0
   // equality rows h = e + D x + E u at the iterate and along the step, and
   // their part of phi, mu h + rho_c / 2 h^2, as a polynomial in a (every lane
   // of a column holds the stage's coefficients); RQ rows per pass, the rows
-  // past p of the last pass read other rows' data (or 0) and are dropped
+  // past p of the last pass repeat row p - 1 (what follows it may be another
+  // instance's, or no data) and are dropped
   float pe0 = 0.f, pe1 = 0.f, pe2 = 0.f;
   if (HQ && p > 0) {   // rows 4 g + s of the lane's stage, summed over the column
     const rsrc_t rh = make_rsrc(ws.hq + (size_t)b * N * 2 * p, N * 2 * p);
@@ -309,7 +310,7 @@ k_trials_mma(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws, int j0
       float ev[RQ], mv[RQ];
 #pragma unroll
       for (int q = 0; q < RQ; ++q) {
-        const int r = r0 + q;
+        const int r = min(r0 + q, p - 1);
 #pragma unroll
         for (int k = 0; k < NT; ++k) Dr[q][k] = vload4<WIDE>(rD, od + r * n + 16 * k, 16 * k + 4 * g, n);
         Er[q] = vload4<WIDE>(rE, oe + r * m, 4 * g, m);

@@ -131,6 +131,25 @@ def _check_evaluation(insts, batch, dtype, off=0):
         assert abs(float(kkt[i]) - rk) <= tol * max(1.0, rk)
 
 
+@pytest.mark.parametrize("layout", ["stage", "pad", "shared"])
+@pytest.mark.parametrize("dtype,model,n,m,p,box", [
+    # wave recursion, matrix-core linearisation, trials and evaluation, adjoint
+    (F32, "tanh", 36, 12, 8, True), (F32, "tanh", 17, 5, 3, False),
+    # tile recursion, row forms
+    (F32, "tanh", 64, 16, 12, True), (F32, "tanh", 52, 20, 3, True),
+    # stage-varying: wave and tile recursion
+    (F32, "ltv", 20, 8, 3, True), (F32, "ltv", 50, 18, 0, True),
+    # FP64 tile recursion
+    (F64, "tanh", 36, 12, 8, True), (F64, "ltv", 20, 7, 2, True),
+])
+def test_layouts(dtype, model, n, m, p, box, layout):
+    print(f"strides {dtype} {model} n={n} m={m} p={p} {layout}", flush=True)
+    insts, batch, keep = _problem(model, dtype, layout, n, m, 18, p, box)
+    off = 1 if layout == "pad" else 0
+    _check_evaluation(insts, batch, dtype, off)
+    _check_iterations(insts, batch, dtype, off, 1 if model == "ltv" else 2)
+
+
 @pytest.mark.parametrize("n,m,N,stride", [
     (12, 4, 17, 2**26 + 4),     # past 4 GiB: 32-bit byte offsets would wrap
     (12, 4, 17, 2**25 + 64),    # past 1 GiB: the offset of absent entries would lie between two stages

@@ -20,7 +20,8 @@ constexpr int kCostateStages = 4;
 
 // One stage's data, lane (g, c): S_t rows 16 i + c, columns 16 k + 4 g + s;
 // dx_t entries 16 k + 4 g + s; dx_t, q_t, s_t, V_t, c_t rows 16 i + c;
-// r_t and du_t of the lane's control 16 g + c (0 for t = N).
+// r_t and du_t of the lane's control 16 g + c (0 for t = N).  whole: S_t is
+// stored whole and read by its rows.
 template <int NT>
 struct CsStage {
   f4 S[NT][NT];
@@ -31,7 +32,7 @@ struct CsStage {
 
 template <int NT, bool WIDE>
 __device__ __forceinline__ void cs_load(CsStage<NT>& d, const Iter<float>& it, const Ws<float>& ws, int b, int t,
-                                        int n, int m, int N, int g, int c) {
+                                        int n, int m, int N, int g, int c, bool whole = false) {
   const size_t st = (size_t)b * (N + 1) + t;
   const rsrc_t rS = make_rsrc(ws.S + st * n * n, n * n);
 #pragma unroll
@@ -44,7 +45,7 @@ __device__ __forceinline__ void cs_load(CsStage<NT>& d, const Iter<float>& it, c
 #pragma unroll
         for (int s = 0; s < 4; ++s) {
           const int r = 16 * k + 4 * g + s, col = 16 * i + c;
-          d.S[i][k][s] = rload(rS, r < n && col < n ? (r * n + col) * 4 : kOOB);
+          d.S[i][k][s] = rload(rS, r < n && col < n ? (whole ? col * n + r : r * n + col) * 4 : kOOB);
         }
       }
     }
@@ -125,14 +126,14 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WIDE ? 
 }
 
 // One stage per wave, for the larger S_t of k_lqr_tile (two buffers of 16 or
-// 25 tiles would spill).
+// 25 tiles would spill), which stores Q_N whole.
 template <int NT, bool WIDE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) k_costate_one(Prob<float> P, Iter<float> it, Ws<float> ws) {
   const int t = blockIdx.x, b = blockIdx.y;
   if (skip_instance(ws, b)) return;
   const int lane = threadIdx.x, g = lane >> 4, c = lane & 15;
   CsStage<NT> d;
-  cs_load<NT, WIDE>(d, it, ws, b, t, P.n, P.m, P.N, g, c);
+  cs_load<NT, WIDE>(d, it, ws, b, t, P.n, P.m, P.N, g, c, t == P.N);
   cs_stage<NT>(d, ws, b, t, P.n, P.N, g, c, lane);
 }
 

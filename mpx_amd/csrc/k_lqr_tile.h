@@ -161,7 +161,8 @@ struct TileLds {
   static constexpr int QV = RD + 16 * MT;        // q by position
   static constexpr int EV = QV + 16 * NT;        // the unit diagonal taken out of A~ (0 or 1) by position
   static constexpr int NONE = EV + 16 * NT;      // what a block has past its matrix lands here, never read
-  static constexpr int TOTAL = NONE + 64;
+  static constexpr int SKEW = NONE + 64;         // whether Q_N is not symmetric
+  static constexpr int TOTAL = SKEW + 4;
 };
 
 // a b over KT k tiles; the even and the odd ones in two chains (half the
@@ -322,9 +323,15 @@ struct TileFactor<double, 1> {
 };
 
 // n + 1 <= 16 NT (NT minimal), 16 (MT - 1) < m <= 16 MT, p <= 16.  Stores K~_t
-// and, with store_s, the upper tiles of S_t and s_t (k_costate_rows).  MODE
-// TILE_CALLER adds the caller's cross Hessian M_t (may be null).
+// and, with store_s, the upper tiles of S_t (Q_N whole) and s_t (k_costate_one).
+// MODE TILE_CALLER adds the caller's cross Hessian M_t (may be null).
 // FP64: m <= 16, n + 1 <= 64, both triangles of S_t.
+//
+// A Q_N that is not symmetric to the bit (a caller's J'WJ) is read by its rows, as
+// k_lqr_seq reads it, which makes stage N - 1 a special one: the columns of S~
+// diag(e) cannot be taken from its rows, so e_j = 0 where column and row j of Q_N
+// differ, and one triangle counts, as there: of H the lower (m <= 16) or the
+// upper one, of P the upper (corrections formed before the loop).
 template <typename T, int NT, int MT, int NW, int MODE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
 k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
@@ -443,11 +450,13 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
     }
     if (tid < 16 * NT) sm[X::QV + tid] = rvq;
   };
-  // after store_data and a barrier: the unit diagonal taken out of A~
-  auto store_diag = [&]() {
+  // after store_data and a barrier: the unit diagonal taken out of A~ (for the
+  // first stage from the columns not marked in its place)
+  auto store_diag = [&](bool first) {
     if (tid < n) {
-      const T e = rdg >= T(0.5) && rdg <= T(2) ? T(1) : T0;
       const int d = tile_pos(tid);
+      const bool keep = first && sm[X::EV + d] != T0;
+      const T e = !keep && rdg >= T(0.5) && rdg <= T(2) ? T(1) : T0;
       sm[X::AT + d * LD + d] = rdg - e;
       sm[X::EV + d] = e;
     }
@@ -527,8 +536,87 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
   load_addends(N - 1);
   store_data();
   lds_sync();
-  store_diag();
+  // where column j of Q_N differs from row j, j is marked in e's place
+#pragma unroll
+  for (int k = 0; k < (256 * NT * NT + NTH - 1) / NTH; ++k) {
+    const int f = tid + k * NTH, i = f / (16 * NT), j = f - i * 16 * NT;
+    if (f < 256 * NT * NT && !(sm[X::S + i * LD + j] == sm[X::S + j * LD + i])) sm[X::EV + j] = sm[X::SKEW] = T(1);
+  }
   lds_sync();
+  store_diag(true);
+  lds_sync();
+
+  auto sb_tile = [&](int u) {   // SB tile u = j NT + i
+    const int j = u / NT, i = u - j * NT;
+    return tile_dot<T, NT>(sm + X::S + 16 * i * LD + (c * LD + 4 * g), sm + X::BT + 16 * j * LD + (c * LD + 4 * g));
+  };
+  auto t_tile = [&](int u) {
+    const int j = u / NT, i = u - j * NT;
+    V4 acc = tile_dot<T, NT>(sm + X::S + 16 * i * LD + (c * LD + 4 * g), sm + X::AT + 16 * j * LD + (c * LD + 4 * g));
+    // + S~ diag(e) (S~ symmetric: its column as a row)
+    const V4 x = O::load_col(sm + X::S + (16 * j + c) * LD + 16 * i, g);
+    const T e = sm[X::EV + 16 * j + c];
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] += e * x[v];
+    return acc;
+  };
+  auto put_t = [&](int u, const V4& x) {
+    const int j = u / NT, i = u - j * NT;
+    O::store_col(sm + X::TT + (16 * j + c) * LD + 16 * i, g, x);
+  };
+  auto put_sb = [&](int u, const V4& x) {
+    const int j = u / NT, i = u - j * NT;
+    O::store_col(sm + X::SBT + (16 * j + c) * LD + 16 * i, g, x);
+  };
+  auto h_tile = [&](int i, int j) {
+    V4 acc = tile_dot<T, NT>(sm + X::BT + 16 * i * LD + (c * LD + 4 * g), sm + X::SBT + 16 * j * LD + (c * LD + 4 * g));
+    if (p > 0) acc += tile_dot<T, 1>(sm + X::ET + 16 * i * LP + (c * LP + 4 * g), sm + X::ET + 16 * j * LP + (c * LP + 4 * g));
+    acc += rv;
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (i == j && O::pos(g, v) == c) acc[v] = 16 * i + pc < m ? acc[v] + sm[X::RD + 16 * i + c] : T(1);
+    return acc;
+  };
+  auto at_tile = [&](int i, int j) {   // A~' T
+    V4 acc = tile_dot<T, NT>(sm + X::AT + 16 * i * LD + (c * LD + 4 * g), sm + X::TT + 16 * j * LD + (c * LD + 4 * g));
+    const V4 x = O::load_col(sm + X::TT + (16 * j + c) * LD + 16 * i, g), e = O::load_col(sm + X::EV + 16 * i, g);
+    return acc + e * x;
+  };
+  // what makes a diagonal tile symmetric from one of its triangles, through buf
+  // (rows of LM)
+  auto one_triangle = [&](const V4& x, T* buf, bool lower) {
+    V4 d;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) buf[O::pos(g, v) * LM + c] = x[v];
+    wave_lds_sync();
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      const int row = O::RG * g + O::RV * v;
+      d[v] = (lower ? row < pc : row > pc) ? buf[c * LM + O::pos(g, v)] - x[v] : T0;
+    }
+    return d;
+  };
+  // Q_N not symmetric: the corrections to stage N - 1's H and P join R and Q (no
+  // branch in the loop: one between H and its factorisation, or beside P, cost 2 %
+  // of a stage)
+  if (__any(sm[X::SKEW] != T0)) {
+    for (int u = w; u < NB; u += NW) put_sb(u, sb_tile(u));
+    for (int u = w; u < NTT; u += NW) put_t(u, t_tile(u));
+    lds_sync();
+    if (w == 0 || (MT == 2 && w == 2)) {
+      const int i = w >> 1;
+      rv += one_triangle(h_tile(i, i), sm + X::Z + 16 * i * LM, MT == 1);
+    }
+    if (w > 0) {
+#pragma unroll
+      for (int s = 0; s < PSL; ++s) {
+        const int i = pij[s] & 15;
+        if (((s + 1) * NWK <= NPM || w - 1 + s * NWK < NPM) && i == pij[s] >> 4)
+          qv[s] += one_triangle(at_tile(i, i), sm + X::WT + 16 * i * LM, false);
+      }
+    }
+    lds_sync();
+  }
 
   for (int t = N - 1; t >= 0; --t) {
     // (pinned to a scalar register: a select into a vector register would make
@@ -543,37 +631,6 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
     };
     phase();
     load_data(tp);
-    auto sb_tile = [&](int u) {   // SB tile u = j NT + i
-      const int j = u / NT, i = u - j * NT;
-      return tile_dot<T, NT>(sm + X::S + 16 * i * LD + (c * LD + 4 * g), sm + X::BT + 16 * j * LD + (c * LD + 4 * g));
-    };
-    auto t_tile = [&](int u) {
-      const int j = u / NT, i = u - j * NT;
-      V4 acc = tile_dot<T, NT>(sm + X::S + 16 * i * LD + (c * LD + 4 * g), sm + X::AT + 16 * j * LD + (c * LD + 4 * g));
-      // + S~ diag(e) (S~ symmetric: its column as a row)
-      const V4 x = O::load_col(sm + X::S + (16 * j + c) * LD + 16 * i, g);
-      const T e = sm[X::EV + 16 * j + c];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) acc[v] += e * x[v];
-      return acc;
-    };
-    auto put_t = [&](int u, const V4& x) {
-      const int j = u / NT, i = u - j * NT;
-      O::store_col(sm + X::TT + (16 * j + c) * LD + 16 * i, g, x);
-    };
-    auto put_sb = [&](int u, const V4& x) {
-      const int j = u / NT, i = u - j * NT;
-      O::store_col(sm + X::SBT + (16 * j + c) * LD + 16 * i, g, x);
-    };
-    auto h_tile = [&](int i, int j) {
-      V4 acc = tile_dot<T, NT>(sm + X::BT + 16 * i * LD + (c * LD + 4 * g), sm + X::SBT + 16 * j * LD + (c * LD + 4 * g));
-      if (p > 0) acc += tile_dot<T, 1>(sm + X::ET + 16 * i * LP + (c * LP + 4 * g), sm + X::ET + 16 * j * LP + (c * LP + 4 * g));
-      acc += rv;
-#pragma unroll
-      for (int v = 0; v < 4; ++v)
-        if (i == j && O::pos(g, v) == c) acc[v] = 16 * i + pc < m ? acc[v] + sm[X::RD + 16 * i + c] : T(1);
-      return acc;
-    };
     // A
     {
       V4 acc[RA];
@@ -796,7 +853,7 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
         }
       }
     }
-    if (t > 0) store_diag();
+    if (t > 0) store_diag(false);
     lds_sync();
   }
 }

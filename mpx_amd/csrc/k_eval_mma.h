@@ -6,9 +6,12 @@
 // lane (g, c).  Entries past a vector's end are read as 0 (not as the next
 // stage's: a NaN there stays in its stage).  The transposed products of the residual, A'V and
 // W'(sech^2 V), read the matrices' columns (64 contiguous bytes per row).  The
-// terminal stage is k_eval_rows'.  Bound by its loads: at B = 1024, 36 x 12 x 50, p = 8 the row
-// form (k_eval_rows), which reads every matrix once per stage, takes 180 us for
-// the model evaluation and 286 us for the residual.
+// block after the last takes the terminal stage (eval_stage; a launch of its own
+// made the smallest evaluations, bound by their launches, slower than the thread
+// per row they replaced: 12 x 12 x 25, B = 1, evaluation and residual 42 us there, 50
+// with a launch more each, 43 now).  Bound by its loads: at B = 1024, 36 x 12 x 50, p
+// = 8 the model evaluation takes 22 us and the residual 47; the row form
+// (k_eval_rows), which reads every matrix once per stage, took 180 and 286.
 #pragma once
 #include "k_eval.h"
 #include "k_lin_mma.h"
@@ -36,6 +39,8 @@ k_eval_mma(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws, float* o
   constexpr bool KKT = WHAT == EVAL_KKT;
   const int b = blockIdx.y, lane = threadIdx.x, g = lane >> 4, c = lane & 15;
   if (WHAT == EVAL_STOP && skip_instance(ws, b)) return;
+  __shared__ float smem[eval_wave_elems<NT>()];
+  if (blockIdx.x == gridDim.x - 1) return eval_stage<float, NT, 1, WHAT, true>(P, prm, it, ws, og, oc, b, P.N, smem);
   const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;
   const int t = blockIdx.x * 16 + c;
   const bool live = t < N;

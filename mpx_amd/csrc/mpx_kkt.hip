@@ -1089,39 +1089,37 @@ mpxkkt_status sqp_iterate_t(hipStream_t st, const mpxkkt_problem* pr, const mpxk
   return s;
 }
 
-// k_eval_rows for n <= 80 (false: the general kernels), after k_eval_mma for the
-// stages t < N where its conditions hold (B = 1024, 36 x 12 x 50, p = 8: model
-// evaluation 180 -> 28 us, KKT residual 286 -> 53 us, a thread per row before
-// 812 and 343 us).  Stages per wave of
-// the row form: one until the stages fill the chip (a wave's stages run one
-// after the other), then four (the instance's matrices stay in L1).
+// k_eval_rows for n <= 80 (false: the general kernels), k_eval_mma where its
+// conditions hold (B = 1024, 36 x 12 x 50, p = 8: model evaluation 180 -> 22 us, KKT
+// residual 286 -> 47 us, a thread per row before 812 and 343 us).  Stages per
+// wave of the row form: one until the stages fill the chip (a wave's stages run
+// one after the other), then four (the instance's matrices stay in L1).
 template <typename T, int WHAT>
 bool eval_rows(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R, const Iter<T>& I,
                const Ws<T>& W, T* g, T* c) {
   if (pr->n > 80) return false;
   const int N1 = pr->horizon + 1;
-  int tbase = 0;
   if constexpr (IsF32<T>::value) {
     const int nt = mma_tiles<T>(pr, 0);
     if (nt) {
       const bool wide = mma_rows16<T>(pr) && al16(I.X) && al16(I.U) && al16(I.V) && al16(c) &&
                         (WHAT != EVAL_KKT || !pr->has_box || al16(I.Ybox));
-      const dim3 grid((pr->horizon + 15) / 16, pr->batch);
+      const dim3 grid((pr->horizon + 15) / 16 + 1, pr->batch);
       with_count<1, 3>(nt, [&](auto k) {
         constexpr int NT = decltype(k)::value;
         if (wide) hipLaunchKernelGGL((k_eval_mma<NT, true, WHAT>), grid, dim3(64), 0, st, P, R, I, W, g, c);
         else hipLaunchKernelGGL((k_eval_mma<NT, false, WHAT>), grid, dim3(64), 0, st, P, R, I, W, g, c);
       });
-      tbase = pr->horizon;
+      return true;
     }
   }
-  const int spw = tbase == 0 && (long long)pr->batch * N1 >= 32768 ? 4 : 1;
-  const dim3 grid((N1 - tbase + kEvalWaves * spw - 1) / (kEvalWaves * spw), pr->batch);
+  const int spw = (long long)pr->batch * N1 >= 32768 ? 4 : 1;
+  const dim3 grid((N1 + kEvalWaves * spw - 1) / (kEvalWaves * spw), pr->batch);
   with_count<1, 5>((pr->n + 15) / 16, [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
     auto go = [&](auto mc) {
       hipLaunchKernelGGL((k_eval_rows<T, NC, decltype(mc)::value, WHAT>), grid, dim3(64 * kEvalWaves), 0, st, P, R, I,
-                         W, g, c, spw, tbase);
+                         W, g, c, spw);
     };
     if (pr->m <= 16) go(std::integral_constant<int, 1>{});
     else go(std::integral_constant<int, 4>{});

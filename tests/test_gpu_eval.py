@@ -66,3 +66,32 @@ def test_nan_stays_in_its_stage(n):
     bad_g, bad_c = torch.isnan(g).cpu().numpy(), torch.isnan(c).any(-1).cpu().numpy()
     assert bad_g.nonzero()[1].tolist() == [7] and not bad_g[1].any()
     assert bad_c.nonzero()[1].tolist() == [7, 8] and not bad_c[1].any()
+
+
+def test_launches():
+    """One launch for the model evaluation, two for the residual (the evaluation and
+    its sum), the terminal stage in the matrix-core form's: evaluations of a few
+    stages are bound by their launches."""
+    import ctypes as C
+    from mpx_amd import _lib as L
+    from mpx_amd.problem import _ptr
+    insts, pts, solver, it = _setup(3, torch.float32, n=12, m=12, N=25, p=0)
+    b = solver.batch
+    g, c = solver.model_eval(it["X"], it["U"])
+    k = solver.kkt(it)
+    ci, ws = b.c_iterate(it), C.c_void_p(solver.ws.data_ptr())
+    hip = C.CDLL("libamdhip64.so")
+    counts = []
+    for what in ("model_eval", "kkt"):
+        graph = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(graph):
+            st = C.c_void_p(torch.cuda.current_stream().cuda_stream)
+            if what == "model_eval":
+                L.check(solver.lib.mpxkkt_model_eval(st, C.byref(b.problem), _ptr(it["X"]), _ptr(it["U"]), _ptr(g), _ptr(c)))
+            else:
+                L.check(solver.lib.mpxkkt_kkt_residual(st, C.byref(b.problem), C.byref(solver.params), C.byref(ci), _ptr(k),
+                                                       ws, solver.ws_bytes))
+        n = C.c_size_t(0)
+        assert hip.hipGraphGetNodes(C.c_void_p(graph.raw_cuda_graph()), None, C.byref(n)) == 0
+        counts.append(n.value)
+    assert counts == [1, 2]

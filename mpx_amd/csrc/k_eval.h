@@ -7,9 +7,9 @@
 // product (columns), which the four groups add once at the end.  A thread per
 // row (the general kernels of k_misc.h, for larger n) reads 64 different cache
 // lines per load and each matrix once per product.  Bound by the L1's rate of
-// loads (about 100 per wave and stage); at B = 1024, 36 x 12 x 50, p = 8 the
-// model evaluation takes 180 us (thread per row: 812), the KKT residual 286 us
-// (343).
+// loads (about 100 per wave and stage); both evaluations at B = 1024: 76 x 32 x 50, p
+// = 12 946 us (four rows in flight 1224, a thread per row 5718), stage-varying
+// 36 x 12 x 33 263 (388, 823), FP64 36 x 12 x 50, p = 8 561 (673, 1475).
 #pragma once
 #include "k_fwd_block.h"
 
@@ -34,7 +34,10 @@ __host__ __device__ constexpr int eval_wave_elems() { return 7 * 16 * NC + 3 * 6
 // The rows of one matrix, four at a time (r0, r0 + 4, ... < rows): f(r0, a), a
 // the lane's entries of row r0 + gq.  Rows past the matrix lie past the
 // descriptor and read 0, columns past it have an offset past every descriptor:
-// no masks.
+// no masks.  Sixteen rows are requested before the first is used: with few
+// stages a wave waits for each request (60 x 20 x 30, B = 1: the two evaluations
+// 16.5 and 20.7 us with four rows in flight, 11.7 and 15.9 with sixteen; a
+// thread per row 17.2 and 13.8).
 template <typename T, int C, typename F>
 __device__ __forceinline__ void eval_rows_of(const T* M, int rows, int cols, int gq, int l, F&& f) {
   typedef TileOps<T> O;
@@ -42,7 +45,17 @@ __device__ __forceinline__ void eval_rows_of(const T* M, int rows, int cols, int
   int off[C];
 #pragma unroll
   for (int j = 0; j < C; ++j) off[j] = l + 16 * j < cols ? (gq * cols + l + 16 * j) * (int)sizeof(T) : kOOB;
-  for (int r0 = 0; r0 < rows; r0 += 4) {
+  int r0 = 0;
+  for (; r0 + 12 < rows; r0 += 16) {
+    T a[4][C];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int j = 0; j < C; ++j) a[k][j] = O::bload(r, off[j], (r0 + 4 * k) * cols * (int)sizeof(T));
+#pragma unroll
+    for (int k = 0; k < 4; ++k) f(r0 + 4 * k, a[k]);
+  }
+  for (; r0 < rows; r0 += 4) {
     T a[C];
 #pragma unroll
     for (int j = 0; j < C; ++j) a[j] = O::bload(r, off[j], r0 * cols * (int)sizeof(T));

@@ -125,7 +125,9 @@ __device__ __forceinline__ void adj_out(const float (&lam)[NT], const float (&xr
   }
 }
 
-// (a wave per instance, one or kWaveBlock of them per block; the waves never meet)
+// (a wave per instance, up to kWaveBlock of them per block; the waves never
+// meet; adjoint_lds bytes of LDS per wave)
+constexpr int adjoint_lds(int nt) { return 2 * nt * nt * 64 * (int)sizeof(f4); }
 template <int NT, bool WIDE>
 __global__ void __launch_bounds__(64 * kWaveBlock)
 k_adjoint_tanh(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws) {
@@ -177,8 +179,8 @@ k_adjoint_tanh(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws) {
   // Q (rows 16 i + c, columns 16 k + 4 g + s) in registers; (I + h A)' and
   // (h kappa W)' in the same layout in LDS, each lane reading back only its
   // own entries
-  __shared__ f4 atws[kWaveBlock][2 * NT * NT * 64];
-  f4* atw = atws[wv];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  f4* atw = reinterpret_cast<f4*>(smem_raw) + wv * 2 * NT * NT * 64;
   f4 Qt[NT][NT];
   {
     f4 At[NT][NT], Wt[NT][NT];

@@ -52,15 +52,17 @@ __device__ __forceinline__ float lane_read(float x, int src) {
 
 // (h kappa W stays in LDS, each lane reading back only its own entries, so
 // that the kernel fits 128 VGPRs: four waves per SIMD, the whole batch of
-// 4096 instances resident at once on 1024 SIMDs; a wave per instance, one or
-// kWaveBlock of them per block, the waves never meet)
+// 4096 instances resident at once on 1024 SIMDs; a wave per instance, up to
+// kWaveBlock of them per block, the waves never meet; fwd_tanh_lds bytes of LDS
+// per wave)
+constexpr int fwd_tanh_lds(int nt) { return nt * nt * 64 * (int)sizeof(f4); }
 template <int NT, bool WIDE, int R>
 __global__ void __launch_bounds__(64 * kWaveBlock) __attribute__((amdgpu_waves_per_eu(WIDE ? 4 : 3)))
 k_fwd_tanh(Prob<float> P, Ws<float> ws) {
-  __shared__ f4 wls[kWaveBlock][NT * NT * 64];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x * (blockDim.x >> 6) + wv;
   if (b >= P.B || skip_instance(ws, b)) return;
-  f4* wl = wls[wv];
+  f4* wl = reinterpret_cast<f4*>(smem_raw) + wv * NT * NT * 64;
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int n = P.n, m = P.m, N = P.N, N1 = N + 1;
   const float hs = P.h, hk = P.h * P.kappa;

@@ -615,11 +615,17 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
       const int nf = fx_in_lqr<T>(pr, R) ? mma_tiles<T>(pr, R.flags) : 0;
       if (nf) {
         const bool wide = mma_rows16<T>(pr) && al16(W.K) && al16(W.cdef) && al16(W.dx);
-        // one wave per block where every instance has a CU's SIMD to itself
-        // anyway, else blocks whose waves sit on different SIMDs (kWaveBlock)
+        // one wave per block where every instance has a CU's SIMD to itself anyway
+        // (and the LDS of one: with four streams of B = 512, 36 x 12 x 50, LDS for four in
+        // every block took a round of iterations from 1195 to 1330 us), else blocks whose
+        // waves sit on different SIMDs (kWaveBlock)
         const int wpb = pr->batch <= kWavesBatch ? 1 : kWaveBlock;
         const dim3 gw((pr->batch + wpb - 1) / wpb), bw(64 * wpb);
-        auto go = [&](auto kern) { hipLaunchKernelGGL(kern, gw, bw, 0, st, P, W); };
+        mpxkkt_status s = MPXKKT_OK;
+        auto go = [&](auto kern) {
+          const size_t lds = (size_t)wpb * fwd_tanh_lds(nf);
+          if ((s = prep_lds(kern, lds)) == MPXKKT_OK) hipLaunchKernelGGL(kern, gw, bw, lds, st, P, W);
+        };
         if (wide) {
           if (nf == 1) go(k_fwd_tanh<1, true, 4>);
           else if (nf == 2) go(k_fwd_tanh<2, true, 4>);
@@ -629,10 +635,12 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
           else if (nf == 2) go(k_fwd_tanh<2, false, 4>);
           else go(k_fwd_tanh<3, false, 2>);
         }
-        mpxkkt_status s = launch_check("k_fwd_tanh");
-        if (s != MPXKKT_OK) return s;
+        if (s != MPXKKT_OK || (s = launch_check("k_fwd_tanh")) != MPXKKT_OK) return s;
         // the costates by the adjoint recursion (k_lqr_wave stored no S_t)
-        auto goa = [&](auto kern) { hipLaunchKernelGGL(kern, gw, bw, 0, st, P, R, I, W); };
+        auto goa = [&](auto kern) {
+          const size_t lds = (size_t)wpb * adjoint_lds(nf);
+          if ((s = prep_lds(kern, lds)) == MPXKKT_OK) hipLaunchKernelGGL(kern, gw, bw, lds, st, P, R, I, W);
+        };
         if (wide) {
           if (nf == 1) goa(k_adjoint_tanh<1, true>);
           else if (nf == 2) goa(k_adjoint_tanh<2, true>);
@@ -642,7 +650,7 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
           else if (nf == 2) goa(k_adjoint_tanh<2, false>);
           else goa(k_adjoint_tanh<3, false>);
         }
-        return launch_check("k_adjoint_tanh");
+        return s != MPXKKT_OK ? s : launch_check("k_adjoint_tanh");
       } else {
         if (NT == 1) fwd_wave<1>(st, gb, cb, (pr->n & 3) == 0, P, W, in);
         else if (NT == 2) fwd_wave<2>(st, gb, cb, (pr->n & 3) == 0, P, W, in);

@@ -478,10 +478,11 @@ __device__ __forceinline__ void il_store_value(const f4 (&S)[NT][NT], const Ws<f
 // and row n's part is added on the vector ALU: column n of S~ A~ gains column
 // n of S~, and row n of A~' (S~ A~) gains row n of S~ A~ (254 instead of 276
 // matrix instructions per stage at n = 36, m = 12, p = 8).
-// A block holds kWaveBlock instances, a wave each, which never meet: the waves
-// of one block sit on different SIMDs.  One-wave blocks were placed by whatever
-// ran before: at 24 x 12 x 100, B = 1024 (a wave per SIMD if spread evenly) the
-// kernel took 348 us behind one predecessor and 508 behind another; this way 350 behind both.
+// A block holds up to kWaveBlock instances, a wave each, which never meet: the
+// waves of one block sit on different SIMDs.  One-wave blocks were placed by
+// whatever ran before: at 24 x 12 x 100, B = 1024 (a wave per SIMD if spread
+// evenly) the kernel took 348 us behind one predecessor and 508 behind another;
+// this way 350 behind both.
 constexpr int kWaveBlock = 4;
 template <int NT, bool CQ, int KSN, bool FA, bool AS>
 __global__ void __launch_bounds__(64 * kWaveBlock, 2) k_lqr_wave(Prob<float> P, Prm<float> prm, Iter<float> it_unused,
@@ -490,7 +491,7 @@ __global__ void __launch_bounds__(64 * kWaveBlock, 2) k_lqr_wave(Prob<float> P, 
   static_assert(!AS || CQ, "the homogeneous step is split off only with the step count of n");
   constexpr int KSS = AS ? KSN - 1 : KSN;   // steps of the last state tile in a contraction over the state
   (void)it_unused;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x * kWaveBlock + wv;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), b = blockIdx.x * (blockDim.x >> 6) + wv;
   if (b >= P.B || skip_instance(ws, b)) return;
   const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
   const int n = P.n, m = P.m, p = P.p, N = P.N, N1 = N + 1;

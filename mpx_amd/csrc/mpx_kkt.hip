@@ -597,6 +597,19 @@ bool fx_in_lqr(const mpxkkt_problem* pr, const Prm<T>& R) {
 // 709 -> 827; 24 x 12 x 50 B = 512 315 -> 282, 1024 351 -> 425.
 constexpr int kWavesBatch = 512;
 
+// Instances (waves) per block of the wave kernels.  Up to kWavesBatch one: each
+// instance has a CU's SIMD to itself anyway, and a block holds the LDS of one
+// (36 x 12 x 50, four streams of B = 512 each: 1330 -> 1195 us a round of iterations with it,
+// LDS for four held before).  Past that blocks, whose waves sit on different
+// SIMDs: three waves while the batch then leaves no CU with a second block or
+// none with a third (256 CUs), else four: of the waves that share a CU the fewer
+// the faster (45 x 14 x 50, blocks of three / four: B = 600 640 / 660, 1100 1005 /
+// 1043, 1500 1062 / 1101; but 900 981 / 706, 2048 1608 / 1188).
+int wave_block(int batch) {
+  if (batch <= kWavesBatch) return 1;
+  return batch <= 3 * 256 || (batch > 4 * 256 && batch <= 6 * 256) ? 3 : kWaveBlock;
+}
+
 // costates, control steps and slope partials: on the wave path the forward
 // pass of the LQR solve and the costates -- for the tanh model after
 // k_linearize_mma k_fwd_tanh and the adjoint sweep k_adjoint_tanh, else
@@ -615,11 +628,7 @@ mpxkkt_status run_fwd_stage(hipStream_t st, const mpxkkt_problem* pr, const Prob
       const int nf = fx_in_lqr<T>(pr, R) ? mma_tiles<T>(pr, R.flags) : 0;
       if (nf) {
         const bool wide = mma_rows16<T>(pr) && al16(W.K) && al16(W.cdef) && al16(W.dx);
-        // one wave per block where every instance has a CU's SIMD to itself anyway
-        // (and the LDS of one: with four streams of B = 512, 36 x 12 x 50, LDS for four in
-        // every block took a round of iterations from 1195 to 1330 us), else blocks whose
-        // waves sit on different SIMDs (kWaveBlock)
-        const int wpb = pr->batch <= kWavesBatch ? 1 : kWaveBlock;
+        const int wpb = wave_block(pr->batch);
         const dim3 gw((pr->batch + wpb - 1) / wpb), bw(64 * wpb);
         mpxkkt_status s = MPXKKT_OK;
         auto go = [&](auto kern) {
@@ -783,9 +792,9 @@ mpxkkt_status run_lqr_wave(hipStream_t st, const mpxkkt_problem* pr, const Prob<
     const int ksn = (pr->n + 1 - 16 * (NT - 1) + 3) / 4;
     const bool cq = P.Q.st == 0 && P.R.st == 0 && in.Bm.st == 0;   // Q, B, R held for the whole recursion
     const dim3 gb(pr->batch);
+    const int wpb = wave_block(pr->batch);
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, dim3((pr->batch + kWaveBlock - 1) / kWaveBlock), dim3(64 * kWaveBlock), 0, st, P, R, I, W,
-                         in);
+      hipLaunchKernelGGL(kern, dim3((pr->batch + wpb - 1) / wpb), dim3(64 * wpb), 0, st, P, R, I, W, in);
     };
     auto gow = [&](auto kern) { hipLaunchKernelGGL(kern, gb, dim3(64 * (NT + 1)), 0, st, P, R, W, in); };
     const bool waves = pr->batch <= kWavesBatch;

@@ -322,9 +322,9 @@ struct TileFactor<double, 1> {
   }
 };
 
-// n + 1 <= 16 NT (NT minimal), 16 (MT - 1) < m <= 16 MT, p <= 16.  Stores K~_t
-// and, with store_s, the upper tiles of S_t (Q_N whole) and s_t (k_costate_one).
-// MODE TILE_CALLER adds the caller's cross Hessian M_t (may be null).
+// n + 1 <= 16 NT (NT minimal), 16 (MT - 1) < m <= 16 MT, p <= 16.  Stores K~_t,
+// the upper tiles of S_t (Q_N whole) and s_t (k_costate_one).  MODE TILE_CALLER
+// adds the caller's cross Hessian M_t (may be null).
 // FP64: m <= 16, n + 1 <= 64, both triangles of S_t.
 //
 // A Q_N that is not symmetric to the bit (a caller's J'WJ) is read by its rows, as
@@ -334,7 +334,7 @@ struct TileFactor<double, 1> {
 // upper one, of P the upper (corrections formed before the loop).
 template <typename T, int NT, int MT, int NW, int MODE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2)))
-k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
+k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in) {
   typedef TileOps<T> O;
   typedef typename O::V4 V4;
   typedef TileLds<T, NT, MT> X;
@@ -519,13 +519,13 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
     for (int e = tid; e < n * n; e += NTH) {
       const int i = e / n, j = e - i * n;
       sm[X::S + tile_pos(i) * LD + tile_pos(j)] = QN[e];
-      if (store_s) pS[(size_t)N * n * n + e] = QN[e];
+      pS[(size_t)N * n * n + e] = QN[e];
     }
     for (int i = tid; i < n; i += NTH) {
       const T q = qN[i];
       sm[X::S + tile_pos(i) * LD + pn] = q;
       sm[X::S + pn * LD + tile_pos(i)] = q;
-      if (store_s) ps[(size_t)N * n + i] = q;
+      ps[(size_t)N * n + i] = q;
     }
   }
   if (bconst && role == 0) {
@@ -821,18 +821,16 @@ k_lqr_tile(Prob<T> P, Prm<T> prm, Ws<T> ws, LqrIn<T> in, int store_s) {
               for (int v = 0; v < 4; ++v) sm[X::S + (16 * i + O::pos(g, v)) * LD + 16 * j + c] = acc[v];
               O::store_col(sm + X::S + (16 * j + c) * LD + 16 * i, g, acc);
             }
-            if (store_s) {
 #pragma unroll
-              for (int v = 0; v < 4; ++v) O::bstore(rS, qo[s], v * srow, acc[v]);
-              if (sizeof(T) == 8 && i != j) {   // both triangles (k_fwd_stage)
-                const int qt = 16 * j + pc < n ? ((16 * j + pc) * n + 16 * i + O::RG * g) * ES : kOOB;
+            for (int v = 0; v < 4; ++v) O::bstore(rS, qo[s], v * srow, acc[v]);
+            if (sizeof(T) == 8 && i != j) {   // both triangles (k_fwd_stage)
+              const int qt = 16 * j + pc < n ? ((16 * j + pc) * n + 16 * i + O::RG * g) * ES : kOOB;
 #pragma unroll
-                for (int v = 0; v < 4; ++v) O::bstore(rS, qt, v * O::RV * ES, acc[v]);
-              }
-              if (j == NT - 1) {
+              for (int v = 0; v < 4; ++v) O::bstore(rS, qt, v * O::RV * ES, acc[v]);
+            }
+            if (j == NT - 1) {
 #pragma unroll
-                for (int v = 0; v < 4; ++v) O::bstore(rs, svo, (16 * i + O::RV * v) * ES, acc[v]);
-              }
+              for (int v = 0; v < 4; ++v) O::bstore(rs, svo, (16 * i + O::RV * v) * ES, acc[v]);
             }
           }
         }

@@ -103,10 +103,11 @@ bool wave_path(const mpxkkt_problem* pr, int flags, int P) {
 // wave kernels do not take.  LQR phase against k_lqr_seq: 76 x 32 x 100 B = 8
 // 6.74 -> 1.13 ms, 76 x 32 x 50 p = 12 B = 256 3.75 -> 0.63 ms, 61 x 12 x 25
 // (caller) B = 64 1.12 -> 0.17 ms.  A caller's problem of one state tile (n <=
-// 15) goes to k_lqr_small (small_path): the quadruped's iterations on clipped
-// penalties amplify a last-digit change of the step to 1e-4 and more of the
-// next iterate (the two product forms of k_lqr_seq, flags bit 0, differ by as
-// much in half of the seeded batches), so its results keep their rounding.
+// 15) goes to k_lqr_small (small_path; with m > 16 it stays on k_lqr_seq): the
+// quadruped's iterations on clipped penalties amplify a last-digit change of the
+// step to 1e-4 and more of the next iterate (the two product forms of k_lqr_seq,
+// flags bit 0, differ by as much in half of the seeded batches), so its results
+// keep their rounding.
 // FP64 (v_mfma_f64): n + 1 <= 64 and m <= 16 (154 KB at the limit): 36 x 12 x 50
 // p = 8 B = 64 524 us (k_lqr_seq: 2690).
 bool tile_path(const mpxkkt_problem* pr, int flags, int P) {
@@ -424,10 +425,15 @@ mpxkkt_status run_lqr_tile(hipStream_t st, const mpxkkt_problem* pr, const Prob<
   auto go = [&](auto nt, auto mt, auto mode) {
     constexpr int NT = decltype(nt)::value, MT = decltype(mt)::value, MODE = decltype(mode)::value;
     constexpr int NW = NT == 1 ? 4 : 8;
-    const size_t lds = (size_t)TileLds<T, NT, MT>::TOTAL * sizeof(T);
-    if ((s = prep_lds(k_lqr_tile<T, NT, MT, NW, MODE>, lds)) != MPXKKT_OK) return;
-    hipLaunchKernelGGL((k_lqr_tile<T, NT, MT, NW, MODE>), dim3(pr->batch), dim3(64 * NW), lds, st, P, R, W, in, 1);
-    s = launch_check("k_lqr_tile");
+    // the others' sizes go elsewhere (tile_path)
+    if constexpr (!IsF32<T>::value || (MODE == TILE_CALLER ? NT > 1 : NT > 3 || MT > 1)) {
+      const size_t lds = (size_t)TileLds<T, NT, MT>::TOTAL * sizeof(T);
+      if ((s = prep_lds(k_lqr_tile<T, NT, MT, NW, MODE>, lds)) != MPXKKT_OK) return;
+      hipLaunchKernelGGL((k_lqr_tile<T, NT, MT, NW, MODE>), dim3(pr->batch), dim3(64 * NW), lds, st, P, R, W, in);
+      s = launch_check("k_lqr_tile");
+    } else {
+      s = fail(MPXKKT_ERR_UNSUPPORTED, "k_lqr_tile is not built for this size");
+    }
   };
   with_count<1, IsF32<T>::value ? 5 : 4>((pr->n + 16) / 16, [&](auto nt) {
     with_count<1, IsF32<T>::value ? 2 : 1>((pr->m + 15) / 16, [&](auto mt) {

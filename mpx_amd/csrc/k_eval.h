@@ -8,8 +8,8 @@
 // row (the general kernels of k_misc.h, for larger n) reads 64 different cache
 // lines per load and each matrix once per product.  Bound by the L1's rate of
 // loads (about 100 per wave and stage); both evaluations at B = 1024: 76 x 32 x 50, p
-// = 12 946 us (four rows in flight 1224, a thread per row 5718), stage-varying
-// 36 x 12 x 33 263 (388, 823), FP64 36 x 12 x 50, p = 8 561 (673, 1475).
+// = 12 700 us (a thread per row 5718), stage-varying 19 x 7 x 33, p = 3 119 (215), FP64
+// 36 x 12 x 50, p = 8 439 (1475).
 #pragma once
 #include "k_fwd_block.h"
 
@@ -84,7 +84,6 @@ __device__ __forceinline__ void eval_stage(const Prob<T>& P, const Prm<T>& prm, 
   const T* V = KKT ? it.V + ((size_t)b * N1 + t) * n : nullptr;
   const T* U = it.U + ((size_t)b * N + (last ? 0 : t)) * m;
   const T* ur = caller || last ? nullptr : P.uref.at(b, t);
-  wave_lds_sync();   // the reads of the stage before
   for (int i = lane; i < LX; i += 64) {
     const bool in = i < n;
     const T x = in ? X[i] : T(0);
@@ -290,19 +289,18 @@ __device__ __forceinline__ void eval_stage(const Prob<T>& P, const Prm<T>& prm, 
   }
 }
 
-// spw consecutive passes of kEvalWaves stages per block, a wave each.
+// kEvalWaves stages per block, a wave each.  (Four stages per wave, one after the
+// other, past 32768 stages: 19 x 7 x 33, stage-varying, B = 1024 135 us against 124,
+// FP64 36 x 12 x 50 558 against 456, 76 x 32 x 50 944 against 725.)
 template <typename T, int NC, int MC, int WHAT>
 __global__ void __launch_bounds__(64 * kEvalWaves)
-k_eval_rows(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws, T* og, T* oc, int spw) {
+k_eval_rows(Prob<T> P, Prm<T> prm, Iter<T> it, Ws<T> ws, T* og, T* oc) {
   __shared__ T smem[kEvalWaves * eval_wave_elems<NC>()];
   const int b = blockIdx.y;
   if (WHAT == EVAL_STOP && skip_instance(ws, b)) return;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  for (int k = 0; k < spw; ++k) {
-    const int t = (blockIdx.x * spw + k) * kEvalWaves + w;
-    if (t > P.N) return;
-    eval_stage<T, NC, MC, WHAT, false>(P, prm, it, ws, og, oc, b, t, smem + w * eval_wave_elems<NC>());
-  }
+  const int t = blockIdx.x * kEvalWaves + w;
+  if (t <= P.N) eval_stage<T, NC, MC, WHAT, false>(P, prm, it, ws, og, oc, b, t, smem + w * eval_wave_elems<NC>());
 }
 
 }  // namespace mpxk

@@ -1114,9 +1114,7 @@ mpxkkt_status sqp_iterate_t(hipStream_t st, const mpxkkt_problem* pr, const mpxk
 
 // k_eval_rows for n <= 80 (false: the general kernels), k_eval_mma where its
 // conditions hold (B = 1024, 36 x 12 x 50, p = 8: model evaluation 180 -> 22 us, KKT
-// residual 286 -> 47 us, a thread per row before 812 and 343 us).  Stages per
-// wave of the row form: one until the stages fill the chip (a wave's stages run
-// one after the other), then four (the instance's matrices stay in L1).
+// residual 286 -> 47 us, a thread per row before 812 and 343 us).
 template <typename T, int WHAT>
 bool eval_rows(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const Prm<T>& R, const Iter<T>& I,
                const Ws<T>& W, T* g, T* c) {
@@ -1136,13 +1134,12 @@ bool eval_rows(hipStream_t st, const mpxkkt_problem* pr, const Prob<T>& P, const
       return true;
     }
   }
-  const int spw = (long long)pr->batch * N1 >= 32768 ? 4 : 1;
-  const dim3 grid((N1 + kEvalWaves * spw - 1) / (kEvalWaves * spw), pr->batch);
+  const dim3 grid((N1 + kEvalWaves - 1) / kEvalWaves, pr->batch);
   with_count<1, 5>((pr->n + 15) / 16, [&](auto nc) {
     constexpr int NC = decltype(nc)::value;
     auto go = [&](auto mc) {
       hipLaunchKernelGGL((k_eval_rows<T, NC, decltype(mc)::value, WHAT>), grid, dim3(64 * kEvalWaves), 0, st, P, R, I,
-                         W, g, c, spw);
+                         W, g, c);
     };
     if (pr->m <= 16) go(std::integral_constant<int, 1>{});
     else go(std::integral_constant<int, 4>{});

@@ -279,8 +279,8 @@ k_trials_mma(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws, int j0
   // equality rows h = e + D x + E u at the iterate and along the step, and
   // their part of phi, mu h + rho_c / 2 h^2, as a polynomial in a (every lane
   // of a column holds the stage's coefficients); RQ rows per pass, the rows
-  // past p of the last pass repeat row p - 1 (what follows it may be another
-  // instance's, or no data) and are dropped
+  // past p of the last pass (what follows may be another instance's, or no data)
+  // are cleared
   float pe0 = 0.f, pe1 = 0.f, pe2 = 0.f;
   if (HQ && p > 0) {   // rows 4 g + s of the lane's stage, summed over the column
     const rsrc_t rh = make_rsrc(ws.hq + (size_t)b * N * 2 * p, N * 2 * p);
@@ -310,12 +310,26 @@ k_trials_mma(Prob<float> P, Prm<float> prm, Iter<float> it, Ws<float> ws, int j0
       float ev[RQ], mv[RQ];
 #pragma unroll
       for (int q = 0; q < RQ; ++q) {
-        const int r = min(r0 + q, p - 1);
+        const int r = r0 + q;
 #pragma unroll
         for (int k = 0; k < NT; ++k) Dr[q][k] = vload4<WIDE>(rD, od + r * n + 16 * k, 16 * k + 4 * g, n);
         Er[q] = vload4<WIDE>(rE, oe + r * m, 4 * g, m);
         ev[q] = rload(re, (int)(tc * P.e.st + r) * 4);
         mv[q] = rload(rmu, (tc * p + r) * 4);
+      }
+      if (r0 + RQ > p) {
+#pragma unroll
+        for (int q = 1; q < RQ; ++q) {
+          const bool in = r0 + q < p;
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+#pragma unroll
+            for (int k = 0; k < NT; ++k) Dr[q][k][v] = in ? Dr[q][k][v] : 0.f;
+            Er[q][v] = in ? Er[q][v] : 0.f;
+          }
+          ev[q] = in ? ev[q] : 0.f;
+          mv[q] = in ? mv[q] : 0.f;
+        }
       }
 #pragma unroll
       for (int q = 0; q < RQ; ++q) {

@@ -9,6 +9,7 @@ import pytest
 
 torch = pytest.importorskip("torch")
 
+from caller_problem import linearization, make_caller_instance, start as caller_start  # noqa: E402
 from mpx_amd import synthetic as syn  # noqa: E402
 from oracle import pdilqr as orc  # noqa: E402
 
@@ -148,6 +149,37 @@ def test_layouts(dtype, model, n, m, p, box, layout):
     off = 1 if layout == "pad" else 0
     _check_evaluation(insts, batch, dtype, off)
     _check_iterations(insts, batch, dtype, off, 1 if model == "ltv" else 2)
+
+
+@pytest.mark.parametrize("layout", ["stage", "pad"])
+@pytest.mark.parametrize("dtype,n,m,p,cross", [(F32, 13, 12, 3, True), (F32, 15, 16, 0, False), (F32, 20, 18, 2, True),
+                                               (F32, 52, 9, 3, True), (F64, 17, 5, 2, False)])
+def test_caller_layouts(dtype, n, m, p, cross, layout):
+    """A caller's linearisation in other layouts: the step's bits of the dense one."""
+    from mpx_amd.caller import CallerBatch, CallerSolver
+    print(f"strides caller {dtype} n={n} m={m} p={p} {layout}", flush=True)
+    insts = [make_caller_instance(i, n=n, m=m, N=6, p=p, box=True) for i in range(2)]
+    st = lambda k: np.stack([d[k] for d in insts])
+    batch = CallerBatch(2, n, m, 6, st("x0"), D=st("D") if p else None, E=st("E") if p else None,
+                        e=st("e") if p else None, ulo=st("ulo"), uhi=st("uhi"), cross=cross, dtype=dtype)
+    starts = [caller_start(d) for d in insts]
+    lins = [linearization(d, s[0], s[1]) for d, s in zip(insts, starts)]
+    lin = {k: np.stack([v[k] for v in lins]) for k in lins[0]}
+    if not cross:
+        del lin["M"]
+    batch.set_linearization(**lin)
+    out, keep = [], []
+    for k in range(2):
+        if k:
+            batch.t = {**batch.t, **batch.lin}
+            for name, x in batch.t.items():
+                if x is not None:
+                    _lay(batch, name, layout, keep)
+        it = batch.iterate_from(*[np.stack([s[j] for s in starts]) for j in range(5)])
+        out.append([x.clone() for x in CallerSolver(batch).direction(it)])
+        torch.cuda.synchronize()
+    for a, b in zip(*out):
+        assert torch.isfinite(a).all() and torch.equal(a, b)
 
 
 @pytest.mark.parametrize("n,m,N,stride", [

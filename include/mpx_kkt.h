@@ -71,7 +71,9 @@ typedef struct {
  * (LTV, TANH): sum_t 1/2 |x_t - xref_t|_Q_t^2 + 1/2 |u_t - uref_t|_R_t^2 +
  * 1/2 |x_N - xref_N|_QN^2 (the Gauss-Newton (Q, R, M = 0) triple of
  * hessian_approx, mpx/utils/objectives.py:75), with optional rows
- * D_t x + E_t u + e_t = 0 and boxes ulo <= u <= uhi.
+ * D_t x + E_t u + e_t = 0 and boxes ulo <= u <= uhi.  Q, R and QN are symmetric
+ * up to rounding: of one that is not, which triangle a kernel reads is
+ * unspecified.
  *
  * MPXKKT_MODEL_CALLER: the caller's dynamics(x, u, t, parameter)
  * (mpx/utils/models.py:6) and cost(W, reference, x, u, t)
@@ -123,20 +125,25 @@ typedef struct {
   int32_t block_threads;  /* threads per block of the per-instance kernels (0 = auto) */
   int32_t trial_group;    /* trials evaluated together (0 = all); 1 if limited_memory */
   int32_t flags;          /* bit 0: FP32 products on VALU instead of the matrix cores;
-                             bit 1: no register-resident wave LQR kernel (FP32,
-                             n + 1 <= 48, m <= 16, n_eq <= 16, one segment);
+                             bit 1: the block LQR kernel instead of those with
+                             operands in registers or LDS tiles (FP32 n + 1 <= 80,
+                             m <= 32; FP64 n + 1 <= 64, m <= 16; n_eq <= 16, one
+                             segment), as bit 0 does too; it keeps the
+                             closed-loop maps, so the workspace is larger;
                              bit 2: single-kernel line search (one block per
                              instance) instead of the stage-parallel one;
                              bit 3: linearisation parallel over stages (lower
-                             latency for small batches; n, m, n_eq <= 64);
+                             latency for small batches; n, m, n_eq <= 64; the
+                             LTV family always takes it);
                              bit 4: the row-per-lane linearisation and
                              line-search trials and the S-based forward pass
                              and costates instead of the matrix-core and
-                             adjoint forms (FP32, tanh model with
-                             stage-invariant A, W, B, Q, R, n <= 48, m <= 16,
-                             n_eq <= 16), and in the wave LQR kernel the
-                             homogeneous offset n on the matrix cores (when
-                             n % 4 == 0 it is otherwise added on the VALU) */
+                             adjoint forms (tanh model with stage-invariant
+                             A, W, B, Q, R: FP32 n <= 80, m <= 32, the FP64
+                             linearisation n <= 64, m <= 16), and in the wave
+                             LQR kernel the homogeneous offset n on the matrix
+                             cores (when n % 4 == 0 it is otherwise added on
+                             the VALU) */
   double hess_floor;      /* pivot floor of the m x m Cholesky factorisations
                              (H_t = R + B'S B, ...): pivot j is raised to
                              hess_floor * |H_jj| when it falls below; keeps
